@@ -678,8 +678,10 @@ bool fp8_dtype(int d) { return d == QG_E4M3 || d == QG_E5M2; }
 // multiple of the 128-wide stage; anything else is packed into workspace.
 struct Fp8Plan {
   bool pack_a, pack_w;
+  bool skinny;    // up to 16 rows: the streaming kernel of skinny_gemm.hip
   bool pingpong;  // large grid: the ping-pong GEMM with fp8 W stages converted in registers
-  int64_t kp;
+  int64_t kp;     // row length of packed operands
+  int64_t ks;     // K of the kernel: k, or kp where both operands are packed
   size_t a_bytes, w_bytes;
   size_t total() const { return a_bytes + w_bytes; }
 };
@@ -688,18 +690,22 @@ Fp8Plan plan_fp8(const void* a, int64_t a_sm, int64_t a_sk, const void* w, int64
                  int64_t m, int64_t n, int64_t k) {
   Fp8Plan pl;
   pl.kp = round_up(k, kStageK);
+  pl.skinny = m <= qg::kSkinnyMaxRows && k > 0;
+  // the streaming kernel takes whole 16-byte chunks of a row, the tiled ones whole stages
+  const int64_t whole = pl.skinny ? 16 : kStageK;
+  pl.ks = k % whole == 0 ? k : pl.kp;
   // In place only when every row's byte offset fits the kernels' 32-bit
   // offsets: the span of the last row ends below 2 GiB.
-  pl.pack_a = !(a_sk == 1 && a_sm % 8 == 0 && aligned16(a) && k % kStageK == 0 &&
+  pl.pack_a = !(a_sk == 1 && a_sm % 8 == 0 && aligned16(a) && k % whole == 0 &&
                 2 * ((m - 1) * a_sm + k) < kMaxOperandBytes);
-  pl.pack_w = !(w_sk == 1 && w_sn % 16 == 0 && aligned16(w) && k % kStageK == 0 &&
+  pl.pack_w = !(w_sk == 1 && w_sn % 16 == 0 && aligned16(w) && k % whole == 0 &&
                 (n - 1) * w_sn + k < kMaxOperandBytes);
   pl.a_bytes = pl.pack_a ? static_cast<size_t>(round_up(2 * m * pl.kp, 256)) : 0;
   pl.w_bytes = pl.pack_w ? static_cast<size_t>(round_up(n * pl.kp, 256)) : 0;
   // >= 192 tiles of 256 x 192 (the INT8 kernel's large-grid rule): the
   // ping-pong GEMM, fp8 W converted exactly to A's 2-byte type in registers
   const int64_t tiles = ((m + 255) / 256) * ((n + 191) / 192);
-  pl.pingpong = tiles >= 192 && 2 * m * pl.kp < kMaxOperandBytes;
+  pl.pingpong = !pl.skinny && tiles >= 192 && 2 * m * pl.kp < kMaxOperandBytes;
   return pl;
 }
 
@@ -746,7 +752,7 @@ extern "C" int qg_fp8w_gemm(const void* a, int a_dtype, int64_t a_sm, int64_t a_
   qg::WdArgs p{};
   p.M = static_cast<int>(m);
   p.N = static_cast<int>(n);
-  p.K = static_cast<int>(pl.kp);
+  p.K = static_cast<int>(pl.ks);
   p.a_f16 = a_dtype == QG_F16;
   if (pl.pack_a) {
     uint16_t* pa = reinterpret_cast<uint16_t*>(ws);
@@ -774,6 +780,22 @@ extern "C" int qg_fp8w_gemm(const void* a, int a_dtype, int64_t a_sm, int64_t a_
   p.bias_dtype = bias_dtype;
   p.out = out;
   p.out_dtype = out_dtype;
+  if (pl.skinny) {
+    qg::SkinnyArgs t{};
+    t.a = p.a;
+    t.a_sm = p.a_sm;
+    t.w = p.w8;
+    t.w_sn = p.w8_sn;
+    t.M = p.M;
+    t.N = p.N;
+    t.K = p.K;
+    t.b_scale = w_scale;
+    t.bias = bias;
+    t.bias_dtype = bias_dtype;
+    t.out = out;
+    t.out_dtype = out_dtype;
+    return qg::launch_skinny_fp8(t, p.a_f16 != 0, p.fp8_e5 != 0, s);
+  }
   if (pl.pingpong && k > 0) {
     // every fp8 value is exact in fp16 and bf16: the 2-byte ping-pong GEMM with
     // the W fragments converted in registers (same fp32 products, order F)

@@ -103,6 +103,21 @@ __device__ __forceinline__ i32x4 fp8x8(uint32_t d0, uint32_t d1) {
   return r;
 }
 
+// Row r of a register is its lanes 16 r .. 16 r + 15 (r < 4). The two-input
+// row exchanges of gfx950:
+//   swap16(a, b): a <- rows (a0, b0, a2, b2), b <- rows (a1, b1, a3, b3)
+//   swap32(a, b): a <- rows (a0, a1, b0, b1), b <- rows (a2, a3, b2, b3)
+__device__ __forceinline__ void swap16(int& a, int& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(a), static_cast<uint32_t>(b), false, false);
+  a = static_cast<int>(r[0]);
+  b = static_cast<int>(r[1]);
+}
+__device__ __forceinline__ void swap32(int& a, int& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(static_cast<uint32_t>(a), static_cast<uint32_t>(b), false, false);
+  a = static_cast<int>(r[0]);
+  b = static_cast<int>(r[1]);
+}
+
 // Compile-time loop: f(std::integral_constant<int, I>) for I in [B, E). Used
 // where every index into a register array must be a constant, independent of
 // the unroller's size heuristics (a dynamic index sends the array to scratch).

@@ -202,6 +202,30 @@ struct WdArgs {
   int out_dtype;
 };
 
+// Few-row GEMM against quantized weights (skinny_gemm.hip, M <= 16): A [M, K]
+// fp16 / bf16 (INT4, fp8) or int8, W [N, K]; unit K strides, 16-byte aligned
+// rows, K a multiple of 16 (INT4: of the group, nk layout).
+struct SkinnyArgs {
+  const void* a;
+  int64_t a_sm;          // elements
+  const void* w;
+  int64_t w_sn;          // bytes
+  int M, N, K;
+  // INT4 storage (see W4Args)
+  int flags, ng, zw;
+  const void* scales;
+  int scale_f32;
+  const void* zeros;
+  const float* b_scale;  // nullptr or per-column [N]
+  const void* bias;      // nullptr or [N]
+  int bias_dtype;
+  void* out;             // [M, N] contiguous
+  int out_dtype;
+  I8GemmArgs i8;         // int8: the epilogue's arguments (the fields above are the operands)
+};
+constexpr int kSkinnyMaxRows = 16;
+hipError_t launch_skinny_fp8(const SkinnyArgs& p, bool f16a, bool e5, hipStream_t stream);
+
 hipError_t launch_wd_w4(const WdArgs& p, hipStream_t stream);
 hipError_t launch_pack_rows_u16(const uint16_t* src, int64_t s_r, int64_t s_k, int64_t rows, int64_t K,
                                 uint16_t* dst, int64_t k_pad, hipStream_t stream);

@@ -1,0 +1,416 @@
+// GEMM of few activation rows (M <= 16) against quantized weights on gfx950:
+// out = A @ W^T with W [N, K] int8 (A int8, dequant epilogues of the INT8
+// GEMM), fp8 e4m3fn / e5m2 or grouped INT4 in the nk layout (A fp16 / bf16).
+//
+// Such a call reads each weight byte once; what bounds it is how many bytes
+// the chip keeps requested, and how many clocks a CU spends on each request.
+//  * A workgroup of 8 waves owns 16 CT output columns and all rows. K is cut
+//    into 128-element chunks; wave w takes chunks w, w + 8, ..., so the
+//    workgroup reads every weight row front to back.
+//  * Each wave copies its chunks (weights, activations, INT4 group
+//    parameters) HBM -> LDS into a ring of its own, D chunks deep, with direct
+//    copies: no barrier until the last one, and every wait is an exact count.
+//    Loading the MFMA fragments into registers instead (16 bytes per lane,
+//    neighbouring lanes in different rows) costs one request per lane, about
+//    72 clocks per KB, whatever the depth in flight: M 16, N 3072, K 12288 fp8
+//    took 19 us that way. A copy's neighbouring lanes read neighbouring bytes.
+//  * A lane reads 16 weight bytes of one column per k-step group and puts them
+//    into K order with two-input row exchanges (swap16 / swap32), so that the
+//    activations are used as they lie in memory.
+//  * LDS rows hold 16-byte chunks permuted by an XOR with the row, chosen so
+//    that the lanes of one ds_read_b128 phase (0-3, 12-15, 20-23, 24-27, and
+//    so on) hit different banks.
+//  * The 8 partial tiles are summed through LDS in wave order.
+// fp8, N 12288, K 3072 (37.7 MB of weights, one box, rotated weight copies):
+// 9.6 us at M 16 and 8.0 us at M <= 4 = 3.9 and 4.7 TB/s, against 40.9 us for
+// the 128-row tiles of k_wd_gemm, whose 96 workgroups walk 24 stages with one
+// stage of lookahead. What is left at M 16 is the copies of the activations
+// (every workgroup reads all of them, about 33 clocks per KB): N 3072, K 12288
+// 13.5 us against 9.1 us at M <= 4.
+#include "qg_common.h"
+#include "qg_epilogue.h"
+#include "qg_internal.h"
+
+namespace qg {
+
+namespace {
+
+enum SkinnyFormat { SK_I8 = 0, SK_E4M3 = 1, SK_E5M2 = 2, SK_W4 = 3, SK_UINT4 = 4 };
+
+// 8 nibbles (K order; high: nibble 7 first) -> 8 fp16 256 + 4 u or bf16 128 + u.
+template <bool F16A>
+struct NibbleExpand {
+  uint32_t sel[4], mask, magic;
+  __device__ __forceinline__ explicit NibbleExpand(bool high) {
+    static_for<0, 4>([&](auto ic) {
+      constexpr uint32_t i = decltype(ic)::value;
+      // halves of register i: elements 2 i and 2 i + 1, from the word (bytes
+      // 0-3) and the word shifted right by 4 (bytes 4-7), 0x0c = zero byte
+      sel[i] = high ? (0x0C000C00u | ((3u - i) << 16) | (7u - i)) : (0x0C000C00u | ((4u + i) << 16) | i);
+    });
+    mask = F16A ? 0x00F000F0u : 0x000F000Fu;
+    magic = F16A ? 0x5C005C00u : 0x43004300u;
+    asm volatile("" : "+v"(mask), "+v"(magic));
+  }
+  __device__ __forceinline__ i32x4 operator()(uint32_t w) const {
+    const uint32_t lo = F16A ? w << 4 : w, hi = F16A ? w : w >> 4;
+    i32x4 r;
+    static_for<0, 4>([&](auto i) {
+      r[int(i)] = static_cast<int>((__builtin_amdgcn_perm(hi, lo, sel[int(i)]) & mask) | magic);
+    });
+    return r;
+  }
+};
+
+template <bool F16A>
+__device__ __forceinline__ f32x4 mfma_half(const i32x4& a, const i32x4& b, const f32x4& c) {
+  if constexpr (F16A)
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
+                                                  0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
+                                                   0, 0);
+}
+
+// RP: activation rows held in LDS (4, 8 or 16 >= M; fragment rows past RP
+// repeat row RP - 1). G: INT4 group size. D: ring depth.
+template <int FMT_, bool F16A_, int RP_, int CT_, int D_, int G_ = 128, int NW_ = 8>
+struct SkinnyCfg {
+  static constexpr int FMT = FMT_, RP = RP_, CT = CT_, D = D_, G = G_;
+  static constexpr bool F16A = F16A_;
+  static constexpr bool I8 = FMT == SK_I8, W4 = FMT >= SK_W4, UINT4 = FMT == SK_UINT4;
+  static constexpr int NW = NW_, KS = 128;
+  static constexpr int AROW = I8 ? KS : 2 * KS;           // LDS bytes of an activation row and chunk
+  static constexpr int WROW = W4 ? KS / 2 : KS;           // of a weight row
+  static constexpr int A_COPIES = RP * AROW / 1024, W_COPIES = 16 * CT * WROW / 1024;
+  static constexpr int SPC = W4 ? KS / G : 0;             // groups per chunk
+  static constexpr int COPIES = A_COPIES + W_COPIES;      // copies of a chunk
+  static constexpr int W_AT = A_COPIES * 1024, STAGE = COPIES * 1024;
+  static constexpr int PITCH = 16 * CT + 1;               // words per row of a partial tile
+  static constexpr int RED = NW * 16 * PITCH * 4;
+  static constexpr int PAR_AT = NW * D * STAGE;           // INT4 group parameters after the rings
+  static constexpr int LDS = PAR_AT > RED ? PAR_AT : RED;
+  static_assert(RP * AROW % 1024 == 0 && A_COPIES >= 1, "activation copies of whole waves");
+  static_assert(D * COPIES < 64 && D >= 2 && D <= 4, "vmcnt range");
+  static_assert(LDS <= 160 * 1024, "LDS per CU");
+};
+
+// LDS words per column of the INT4 scales and zero points: odd, so that a
+// group's 16 columns lie in different banks. bf16 scales of a column may start
+// in the upper half of a word.
+__host__ __device__ __forceinline__ int skinny_scale_pitch(int ng, bool f32) { return (f32 ? ng : ng / 2 + 1) | 1; }
+__host__ __device__ __forceinline__ int skinny_zero_pitch(int ng, int zw, bool packed) { return (packed ? zw : ng) | 1; }
+inline int skinny_par_bytes(const SkinnyArgs& p, int cols) {
+  const int s = cols * skinny_scale_pitch(p.ng, p.scale_f32);
+  const int z = cols * skinny_zero_pitch(p.ng, p.zw, p.flags & QG_W4_ZEROS_PACKED);
+  return 4 * (((s + 63) & ~63) + ((z + 63) & ~63));
+}
+
+template <typename C>
+__global__ __launch_bounds__(64 * C::NW) void k_skinny_gemm(SkinnyArgs p) {
+#pragma clang fp contract(off)
+  using acc_t = std::conditional_t<C::I8, i32x4, f32x4>;
+  constexpr int CT = C::CT, D = C::D;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, q = lane >> 4;
+  const int n0 = blockIdx.x * 16 * CT;
+  char* const ring = smem + wave * D * C::STAGE;
+  const uint32_t ring_addr = lds_addr_of(ring);
+
+  // ---- copy plan: per-lane byte offsets from the operand bases -------------
+  // Copy i of the activations covers 1024 / AROW rows; lane l lands in 16-byte
+  // slot l of it and fetches the chunk that the row's XOR stores there.
+  constexpr int APC = 1024 / C::AROW, ASL = C::AROW / 16;  // rows per copy, slots per row
+  constexpr int WPC = 1024 / C::WROW, WSL = C::WROW / 16;
+  uint32_t aoff[C::A_COPIES], woff[C::W_COPIES];
+  auto a_xor = [&](int row) __attribute__((always_inline)) { return C::I8 ? 2 * ((row >> 1) & 3) : (row & 15); };
+  auto w_xor = [&](int c) __attribute__((always_inline)) { return C::W4 ? (-(c >> 2)) & 3 : 2 * ((c >> 1) & 3); };
+  const int a_slot = lane % ASL, w_slot = lane % WSL;
+  static_for<0, C::A_COPIES>([&](auto i) {
+    const int row = APC * i + lane / ASL;
+    aoff[i] = static_cast<uint32_t>(min(row, p.M - 1)) * static_cast<uint32_t>((C::I8 ? 1 : 2) * p.a_sm);
+  });
+  static_for<0, C::W_COPIES>([&](auto i) {
+    const int c = WPC * i + lane / WSL;
+    woff[i] = static_cast<uint32_t>(min(n0 + c, p.N - 1)) * static_cast<uint32_t>(p.w_sn);
+  });
+  const uint32_t a_end = static_cast<uint32_t>((C::I8 ? 1 : 2) * p.K) - 16;  // last 16 bytes of a row
+  const uint32_t w_end = static_cast<uint32_t>(C::W4 ? p.K / 2 : p.K) - 16;
+  const int chunks = (p.K + C::KS - 1) / C::KS;
+  auto issue = [&](int c, int slot) __attribute__((always_inline)) {
+    const uint32_t at = ring_addr + slot * C::STAGE;
+    static_for<0, C::W_COPIES>([&](auto i) {
+      const int r = (WPC * i + lane / WSL) & 15;
+      const uint32_t k = static_cast<uint32_t>(C::WROW) * c + 16u * (w_slot ^ w_xor(r));
+      dma16s_nt(p.w, woff[i] + min(k, w_end), at + C::W_AT + 1024 * i);
+    });
+    static_for<0, C::A_COPIES>([&](auto i) {
+      const int r = APC * i + lane / ASL;
+      const uint32_t k = static_cast<uint32_t>(C::AROW) * c + 16u * (a_slot ^ a_xor(r));
+      dma16s(p.a, aoff[i] + min(k, a_end), at + 1024 * i);
+    });
+  };
+  // INT4: the scales and zero points of the workgroup's columns are contiguous
+  // (rows n0 .. of [N, ng] / [N, zw]): copied as dwords by all waves before
+  // anything else. One copy per column, group and chunk instead (64 scattered
+  // dwords) costs more clocks than the chunk's weights (M 16, N 4096, K 14336:
+  // 19 us).
+  const bool zpacked = C::UINT4 || (p.flags & QG_W4_ZEROS_PACKED);
+  const bool sf32 = !C::UINT4 && p.scale_f32;
+  const int sper = skinny_scale_pitch(p.ng, sf32), zper = skinny_zero_pitch(p.ng, p.zw, zpacked);
+  const int spart = (16 * CT * sper + 63) & ~63;  // words of the scale part
+  if constexpr (C::W4) {
+    const uint32_t par_addr = lds_addr_of(smem + C::PAR_AT);
+    // word e: word e % pitch of column e / pitch (padding re-reads a word that exists)
+    auto copy_words = [&](const void* base, int pitch, int used, uint32_t at, auto first)
+        __attribute__((always_inline)) {
+      for (int w0 = 64 * wave; w0 < 16 * CT * pitch; w0 += 64 * C::NW) {
+        const int e = w0 + lane, cc = e / pitch, k = min(e - cc * pitch, used - 1);
+        dma4s(base, 4u * (first(static_cast<uint32_t>(min(n0 + cc, p.N - 1))) + k), at + 4 * w0);
+      }
+    };
+    // the words of a column's bf16 scales start at the one holding group 0
+    const uint32_t ng = p.ng;
+    const int sused = sf32 ? p.ng : (p.ng + 1) / 2;
+    copy_words(p.scales, sper, sused, par_addr, [&](uint32_t n) { return sf32 ? n * ng : (n * ng) >> 1; });
+    copy_words(p.zeros, zper, zpacked ? p.zw : p.ng, par_addr + 4 * spart,
+               [&](uint32_t n) { return n * static_cast<uint32_t>(zpacked ? p.zw : p.ng); });
+  }
+
+  acc_t acc[CT];
+  f32x4 total[C::W4 ? CT : 1];
+  static_for<0, CT>([&](auto t) {
+    acc[t] = acc_t{0, 0, 0, 0};
+    if constexpr (C::W4) total[t] = f32x4{0, 0, 0, 0};
+  });
+  const NibbleExpand<C::F16A> expand(C::W4 && !C::UINT4 && (p.flags & QG_W4_ORDER_HIGH));
+  const uint32_t wxor = (C::W4 && !C::UINT4 && (p.flags & QG_W4_SIGNED_NIBBLES)) ? 0x88888888u : 0u;
+  uint32_t one2 = C::F16A ? 0x3C003C00u : 0x3F803F80u;
+  asm volatile("" : "+v"(one2));
+  const i32x4 ones = {static_cast<int>(one2), static_cast<int>(one2), static_cast<int>(one2), static_cast<int>(one2)};
+  const int arow = min(col, C::RP - 1);
+
+  // tail: the chunk holds K elements past the end, which are zeroed (byte
+  // formats; INT4 groups past the end get scale 0)
+  auto compute = [&](int c, int slot, bool tail) __attribute__((always_inline)) {
+    const char* const st = ring + slot * C::STAGE;
+    auto a_frag = [&](int chunk) __attribute__((always_inline)) {
+      return *reinterpret_cast<const i32x4*>(st + arow * C::AROW + 16 * (chunk ^ a_xor(arow)));
+    };
+    auto w_frag = [&](int t, int chunk) __attribute__((always_inline)) {
+      return *reinterpret_cast<const i32x4*>(st + C::W_AT + (16 * t + col) * C::WROW + 16 * (chunk ^ w_xor(col)));
+    };
+    const i32x4 zero4 = {0, 0, 0, 0};
+    if constexpr (C::I8) {
+      static_for<0, 2>([&](auto u) {
+        const bool in = !tail || C::KS * c + 64 * u + 16 * q < p.K;
+        const i32x4 a = in ? a_frag(4 * u + q) : zero4;
+        static_for<0, CT>([&](auto t) {
+          acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, w_frag(t, 4 * u + q), acc[t], 0, 0, 0);
+        });
+      });
+    } else if constexpr (!C::W4) {
+      static_for<0, 2>([&](auto u) {
+        i32x4 w[CT];
+        static_for<0, CT>([&](auto t) {
+          w[t] = w_frag(t, 4 * u + q);
+          if (tail && C::KS * c + 64 * u + 16 * q >= p.K) w[t] = zero4;
+          // 16 q .. 16 q + 15 -> 32 h + 8 q .. + 7 for step h
+          int w0 = w[t][0], w1 = w[t][1], w2 = w[t][2], w3 = w[t][3];
+          swap16(w0, w2);
+          swap32(w0, w2);
+          swap16(w1, w3);
+          swap32(w1, w3);
+          w[t] = i32x4{w0, w1, w2, w3};
+        });
+        static_for<0, 2>([&](auto h) {
+          constexpr int H = decltype(h)::value;
+          const bool in = !tail || C::KS * c + 64 * u + 32 * H + 8 * q < p.K;
+          const i32x4 a = in ? a_frag(8 * u + 4 * H + q) : zero4;
+          static_for<0, CT>([&](auto t) {
+            const i32x4 b = fp8x8<C::F16A, C::FMT == SK_E5M2>(static_cast<uint32_t>(w[t][2 * H]),
+                                                              static_cast<uint32_t>(w[t][2 * H + 1]));
+            acc[t] = mfma_half<C::F16A>(a, b, acc[t]);
+          });
+        });
+      });
+    } else {
+      constexpr int SPG = 4 / C::SPC;  // k-steps per group
+      constexpr float MAGIC = C::F16A ? 256.0f : 128.0f, UNIT = C::F16A ? 4.0f : 1.0f;
+      const char* const par = smem + C::PAR_AT;
+      const uint32_t* const zpar = reinterpret_cast<const uint32_t*>(par) + spart;
+      i32x4 w[CT];
+      static_for<0, CT>([&](auto t) {
+        w[t] = w_frag(t, q);
+        // words 4 q + j -> 4 j + q
+        int w0 = w[t][0], w1 = w[t][1], w2 = w[t][2], w3 = w[t][3];
+        swap16(w0, w1);
+        swap16(w2, w3);
+        swap32(w0, w2);
+        swap32(w1, w3);
+        w[t] = i32x4{w0, w1, w2, w3};
+      });
+      f32x4 asum = {0, 0, 0, 0};
+      static_for<0, 4>([&](auto j) {
+        constexpr int J = decltype(j)::value;
+        if constexpr (J % SPG == 0) {
+          asum = f32x4{0, 0, 0, 0};
+          static_for<0, CT>([&](auto t) { acc[t] = acc_t{0, 0, 0, 0}; });
+        }
+        const i32x4 a = a_frag(4 * J + q);
+        asum = mfma_half<C::F16A>(a, ones, asum);
+        // steps 0 .. 3 of the exchanged words: w0, w1 hold words 0-3 and 4-7,
+        // w2, w3 words 8-11 and 12-15
+        static_for<0, CT>([&](auto t) {
+          acc[t] = mfma_half<C::F16A>(a, expand(static_cast<uint32_t>(w[t][J]) ^ wxor), acc[t]);
+        });
+        if constexpr (J % SPG == SPG - 1) {
+          constexpr int gi = J / SPG;
+          const int g = c * C::SPC + gi;
+          static_for<0, CT>([&](auto t) {
+            const int cc = 16 * t + col, gl = min(g, p.ng - 1);
+            const uint32_t odd = static_cast<uint32_t>(min(n0 + cc, p.N - 1)) * p.ng & 1u;  // of the first bf16 scale
+            const float sc = sf32 ? reinterpret_cast<const float*>(par)[cc * sper + gl]
+                                  : bf16_to_f32(reinterpret_cast<const uint16_t*>(par)[cc * 2 * sper + odd + gl]);
+            const float s = g < p.ng ? sc / UNIT : 0.0f;
+            const uint32_t rz = zpacked ? zpar[cc * zper + (gl >> 3)] : zpar[cc * zper + gl];
+            const int z = zpacked ? static_cast<int>((rz >> (4 * (gl & 7))) & 15u) : static_cast<int>(rz);
+            const int zu = (!C::UINT4 && (p.flags & QG_W4_SIGNED_NIBBLES)) ? (zpacked ? (z ^ 8) : z + 8) : z;
+            const float zb = MAGIC + UNIT * static_cast<float>(zu);
+            static_for<0, 4>([&](auto e) {
+              const float v = __builtin_fmaf(-zb, asum[int(e)], acc[t][int(e)]);
+              total[t][int(e)] = __builtin_fmaf(s, v, total[t][int(e)]);
+            });
+          });
+        }
+      });
+    }
+  };
+
+  // ---- this wave's chunks --------------------------------------------------
+  const int n = chunks > wave ? (chunks - wave + C::NW - 1) / C::NW : 0;
+  static_for<0, D>([&](auto d) {
+    if (d < n) issue(wave + C::NW * d, d);
+  });
+  if constexpr (C::W4) {  // the parameters have landed (the chunks may still fly)
+    if (n >= D) wait_vm_barrier<D * C::COPIES>();
+    else wait_vm_barrier<0>();
+  }
+  const bool ragged = p.K % C::KS != 0;
+  int slot = 0;
+  for (int i = 0; i < n; ++i) {
+    const int after = n - 1 - i;  // chunks issued after this one: min(after, D - 1)
+    if (after >= D - 1) wait_vm<(D - 1) * C::COPIES>();
+    else if (D > 2 && after == D - 2) wait_vm<(D > 2 ? D - 2 : 0) * C::COPIES>();
+    else if (D > 3 && after == D - 3) wait_vm<(D > 3 ? D - 3 : 0) * C::COPIES>();
+    else wait_vm<0>();
+    const int c = wave + C::NW * i;
+    if (!C::W4 && ragged && c == chunks - 1) compute(c, slot, true);
+    else compute(c, slot, false);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot's reads are done
+    if (i + D < n) issue(c + C::NW * D, slot);
+    slot = slot + 1 == D ? 0 : slot + 1;
+  }
+
+  // ---- partial tiles: row 4 q + i, column 16 t + col -------------------------
+  uint32_t* const red = reinterpret_cast<uint32_t*>(smem);
+  __syncthreads();  // every ring is done with
+  static_for<0, CT>([&](auto t) {
+    static_for<0, 4>([&](auto i) {
+      uint32_t v;
+      if constexpr (C::W4) v = __float_as_uint(total[t][int(i)]);
+      else if constexpr (C::I8) v = static_cast<uint32_t>(acc[t][int(i)]);
+      else v = __float_as_uint(acc[t][int(i)]);
+      red[(wave * 16 + 4 * q + i) * C::PITCH + 16 * t + col] = v;
+    });
+  });
+  __syncthreads();
+  for (int e = threadIdx.x; e < C::RP * 16 * CT; e += 64 * C::NW) {
+    const int row = e / (16 * CT), cc = e % (16 * CT);
+    const int nn = n0 + cc;
+    if (row >= p.M || nn >= p.N) continue;
+    if constexpr (C::I8) {
+      int v = static_cast<int>(red[row * C::PITCH + cc]);
+#pragma unroll
+      for (int w = 1; w < C::NW; ++w) v += static_cast<int>(red[(w * 16 + row) * C::PITCH + cc]);
+      i8_store_out(p.i8, row, nn, v);
+    } else {
+      const int64_t idx = static_cast<int64_t>(row) * p.N + nn;
+      float v = __uint_as_float(red[row * C::PITCH + cc]);
+#pragma unroll
+      for (int w = 1; w < C::NW; ++w) v = v + __uint_as_float(red[(w * 16 + row) * C::PITCH + cc]);
+      if (!C::W4 && p.b_scale) v = v * p.b_scale[nn];
+      if (p.bias) v = v + bias_value(load_bias_bits(p.bias, p.bias_dtype, nn), p.bias_dtype);
+      if (p.out_dtype == QG_F32) store_elem<QG_F32>(p.out, idx, __float_as_uint(v));
+      else if (p.out_dtype == QG_F16) store_elem<QG_F16>(p.out, idx, f32_to_f16(v));
+      else store_elem<QG_BF16>(p.out, idx, f32_to_bf16(v));
+    }
+  }
+}
+
+template <typename C>
+hipError_t launch_skinny_c(const SkinnyArgs& p, hipStream_t stream) {
+  int lds = C::LDS;
+  if constexpr (C::W4) {
+    const int with_par = C::PAR_AT + skinny_par_bytes(p, 16 * C::CT);
+    lds = with_par > lds ? with_par : lds;
+  }
+  hipLaunchKernelGGL(k_skinny_gemm<C>, dim3(ceil_div(p.N, 16 * C::CT)), dim3(64 * C::NW), lds, stream, p);
+  return hipGetLastError();
+}
+
+constexpr int kCUs = 256;  // MI355X
+constexpr int kMaxLds = 160 * 1024;
+
+// Column tiles per workgroup: the copies a CU issues decide the time once the
+// weights are in flight, ceil(workgroups / CUs) x (activation copies + CT x
+// weight copies) of a chunk; the smallest CT among equals. fp8, M 16, K 3072:
+// N 12288 13.2 / 12.2 / 9.6 us with 1 / 2 / 3 tiles (18 / 16 / 10 by this
+// count), N 3072 5.3 / 6.3 / 7.7 us (6 / 8 / 10).
+int skinny_tiles(int n, int a_copies, int w_copies, int max_tiles, const int* allowed, int count) {
+  int best = allowed[0];
+  long best_cost = -1;
+  for (int i = 0; i < count && allowed[i] <= max_tiles; ++i) {
+    const int ct = allowed[i];
+    const long groups = ceil_div(n, 16 * ct);
+    const long cost = (groups + kCUs - 1) / kCUs * (a_copies + ct * w_copies);
+    if (best_cost < 0 || cost < best_cost) {
+      best = ct;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+// Ring depth 2: the 8 waves of a workgroup keep 48 to 160 KB in flight, and
+// depths 3 and 4 measured the same or slower (fewer workgroups per CU).
+template <int FMT, bool F16A, int RP>
+hipError_t launch_skinny_bytes(const SkinnyArgs& p, hipStream_t stream) {
+  using C1 = SkinnyCfg<FMT, F16A, RP, 1, 2>;
+  const int allowed[] = {1, 2, 3};
+  switch (skinny_tiles(p.N, C1::A_COPIES, C1::W_COPIES, 3, allowed, 3)) {
+    case 1: return launch_skinny_c<C1>(p, stream);
+    case 2: return launch_skinny_c<SkinnyCfg<FMT, F16A, RP, 2, 2>>(p, stream);
+    default: return launch_skinny_c<SkinnyCfg<FMT, F16A, RP, 3, 2>>(p, stream);
+  }
+}
+
+template <int FMT, bool F16A>
+hipError_t launch_skinny_fp8_rows(const SkinnyArgs& p, hipStream_t stream) {
+  if (p.M <= 4) return launch_skinny_bytes<FMT, F16A, 4>(p, stream);
+  if (p.M <= 8) return launch_skinny_bytes<FMT, F16A, 8>(p, stream);
+  return launch_skinny_bytes<FMT, F16A, 16>(p, stream);
+}
+
+}  // namespace
+
+hipError_t launch_skinny_fp8(const SkinnyArgs& p, bool f16a, bool e5, hipStream_t stream) {
+  if (p.M < 1 || p.M > kSkinnyMaxRows || p.K % 16 != 0 || p.K < 16) return hipErrorInvalidValue;
+  if (f16a) return e5 ? launch_skinny_fp8_rows<SK_E5M2, true>(p, stream) : launch_skinny_fp8_rows<SK_E4M3, true>(p, stream);
+  return e5 ? launch_skinny_fp8_rows<SK_E5M2, false>(p, stream) : launch_skinny_fp8_rows<SK_E4M3, false>(p, stream);
+}
+
+}  // namespace qg

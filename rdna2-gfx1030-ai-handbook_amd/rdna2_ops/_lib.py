@@ -150,6 +150,12 @@ def ws_ptr(ws: torch.Tensor | None):
     return ctypes.c_void_p(aligned), ws.numel() - (aligned - addr)
 
 
+def skinny_tiles(n: int, a_copies: int, w_copies: int, allowed=(1, 2, 3)) -> int:
+    """Column tiles of 16 per workgroup of the few-row kernel, as skinny_tiles
+    in csrc/skinny_gemm.hip picks them."""
+    return min(allowed, key=lambda ct: (-(-(-(-n // (16 * ct))) // 256) * (a_copies + ct * w_copies), ct))
+
+
 @functools.lru_cache(maxsize=1)
 def kernel_resources() -> dict:
     path = library_path().with_name("kernel_resources.json")

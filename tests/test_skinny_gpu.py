@@ -1,0 +1,69 @@
+"""The few-row (M <= 16) streaming kernel on the GPU: the edges of its row
+counts, column tiles and K chunks, each weight format against its oracle."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import case
+from oracle import fp8 as o8
+from test_fp8_gpu import check, codes_tensor
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("e5", [False, True])
+@pytest.mark.parametrize("adtype", [torch.bfloat16, torch.float16])
+def test_fp8_one_hot_rows(cuda, e5, adtype):
+    """One-hot activation rows read every K position of a whole chunk, a
+    second one and a 16-element tail back exactly: the K order of A and W."""
+    from rdna2_ops.fp8_weight_gemm_v06 import fp8_weight_gemm
+    case(f"skinny fp8 one-hot e5={e5} {adtype}")
+    codes = np.arange(256, dtype=np.uint8)
+    codes = codes[np.isfinite(o8.decode_bits(codes, e5))]
+    n, k = 37, 272
+    w = codes[(np.arange(n)[:, None] * 7 + np.arange(k)[None, :]) % len(codes)].astype(np.uint8)
+    dec = o8.decode_bits(w, e5)
+    wt = codes_tensor(w, e5, cuda)
+    for k0 in range(0, k, 16):
+        a = torch.zeros(16, k, dtype=adtype)
+        a[torch.arange(16), k0 + torch.arange(16)] = 1
+        y = fp8_weight_gemm(a.to(cuda), wt, method="fused_dot2")
+        assert np.array_equal(y.float().cpu().numpy(), dec[:, k0:k0 + 16].T.astype(np.float32)), k0
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 1, 16), (2, 16, 128), (4, 17, 144), (5, 33, 1024), (8, 47, 1040), (9, 48, 2064), (16, 4097, 256),
+    (16, 768, 3072), (3, 8208, 384), (7, 12304, 160), (16, 20, 8), (11, 31, 257),
+])
+@pytest.mark.parametrize("e5,adtype", [(False, torch.bfloat16), (True, torch.float16)])
+def test_fp8_shapes(cuda, m, n, k, e5, adtype):
+    """Rows, column tiles of one to three, chunks past a wave's first, tails
+    and (K % 16 != 0) packed operands; scale and bias; strided activations."""
+    from rdna2_ops.fp8_weight_gemm_v06 import fp8_weight_gemm
+    case(f"skinny fp8 {m}x{n}x{k} e5={e5} {adtype}")
+    rng = np.random.default_rng(m * 1000 + n + k)
+    codes = rng.integers(0, 256, (n, k)).astype(np.uint8)
+    bad = ~np.isfinite(o8.decode_bits(codes, e5)) | (np.abs(o8.decode_bits(codes, e5)) > 4)
+    codes[bad] = 0x30
+    a = torch.from_numpy(rng.standard_normal((m, k + 8)).astype(np.float32)).to(adtype)
+    scale = torch.from_numpy(rng.uniform(0.5, 2, n).astype(np.float32))
+    bias = torch.from_numpy(rng.standard_normal(n).astype(np.float32)).to(adtype)
+    ac = a.to(cuda)[:, :k]
+    y = fp8_weight_gemm(ac, codes_tensor(codes, e5, cuda), bias=bias.to(cuda), method="fused_dot2",
+                        w_scale=scale.to(cuda))
+    a64, w64 = a[:, :k].double().numpy(), o8.decode_bits(codes, e5).astype(np.float64)
+    s64, b64 = scale.double().numpy(), bias.double().numpy()
+    check(y, (a64 @ w64.T) * s64 + b64, (np.abs(a64) @ np.abs(w64).T) * s64 + np.abs(b64), adtype, "skinny fp8")
+
+
+def test_fp8_values_past_k(cuda):
+    """Weight bytes after the last K element of a row (the next row's, here
+    NaN codes) do not reach the result."""
+    from rdna2_ops.fp8_weight_gemm_v06 import fp8_weight_gemm
+    case("skinny fp8 NaN past K")
+    n, k, pitch = 24, 144, 256
+    store = np.full((n, pitch), 0x7f, np.uint8)
+    store[:, :k] = 0x38  # 1.0
+    w = codes_tensor(store, False, cuda)[:, :k]
+    y = fp8_weight_gemm(torch.ones(3, k, dtype=torch.bfloat16, device=cuda), w, method="fused_dot2")
+    assert torch.equal(y.float().cpu(), torch.full((3, n), float(k)))
