@@ -225,6 +225,9 @@ struct SkinnyArgs {
 };
 constexpr int kSkinnyMaxRows = 16;
 hipError_t launch_skinny_fp8(const SkinnyArgs& p, bool f16a, bool e5, hipStream_t stream);
+// nk layout, M <= 16, group parameters that fit in LDS.
+bool skinny_w4_applies(const W4Args& p);
+hipError_t launch_skinny_w4(const W4Args& p, hipStream_t stream);
 
 hipError_t launch_wd_w4(const WdArgs& p, hipStream_t stream);
 hipError_t launch_pack_rows_u16(const uint16_t* src, int64_t s_r, int64_t s_k, int64_t rows, int64_t K,

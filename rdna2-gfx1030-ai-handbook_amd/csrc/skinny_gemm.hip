@@ -405,7 +405,90 @@ hipError_t launch_skinny_fp8_rows(const SkinnyArgs& p, hipStream_t stream) {
   return launch_skinny_bytes<FMT, F16A, 16>(p, stream);
 }
 
+// INT4 column tiles: four pay only at 16 rows (uint4, N 14336, K 4096: 19 / 14
+// / 17 / 12 us with 1 / 2 / 3 / 4), one or two below; up to K 512, where half
+// of the waves have no chunk and every choice takes 3 to 4 us, as many as the
+// registers of a wide workgroup allow. The parameters of K / G groups have to
+// fit next to the rings.
+template <typename C1>
+int skinny_w4_tiles(const SkinnyArgs& p) {
+  int ct;
+  if (p.K <= 512) {
+    ct = C1::RP == 4 ? 2 : C1::G == 128 ? 4 : C1::G == 64 ? 2 : 1;
+  } else {
+    const int allowed[] = {1, 2, 4};
+    ct = skinny_tiles(p.N, C1::A_COPIES, C1::W_COPIES, C1::RP == 16 && C1::G != 32 ? 4 : 2, allowed, 3);
+  }
+  while (ct > 1 && C1::RP * 4096 + ct * 16384 + skinny_par_bytes(p, 16 * ct) > kMaxLds) ct >>= 1;
+  return ct;
+}
+
+template <int FMT, bool F16A, int RP, int G>
+hipError_t launch_skinny_w4_rows(const SkinnyArgs& p, hipStream_t stream) {
+  using C1 = SkinnyCfg<FMT, F16A, RP, 1, 2, G>;
+  const int ct = skinny_w4_tiles<C1>(p);
+  if (C1::PAR_AT + skinny_par_bytes(p, 16) > kMaxLds) return hipErrorInvalidValue;
+  if constexpr (RP > 4 && G != 32) {
+    if (ct == 4) return launch_skinny_c<SkinnyCfg<FMT, F16A, RP, 4, 2, G>>(p, stream);
+  }
+  if (ct == 2) return launch_skinny_c<SkinnyCfg<FMT, F16A, RP, 2, 2, G>>(p, stream);
+  return launch_skinny_c<C1>(p, stream);
+}
+
+template <int FMT, bool F16A, int G>
+hipError_t launch_skinny_w4_g(const SkinnyArgs& p, hipStream_t stream) {
+  if (p.M <= 4) return launch_skinny_w4_rows<FMT, F16A, 4, G>(p, stream);
+  if (p.M <= 8) return launch_skinny_w4_rows<FMT, F16A, 8, G>(p, stream);
+  return launch_skinny_w4_rows<FMT, F16A, 16, G>(p, stream);
+}
+
+template <bool F16A>
+hipError_t launch_skinny_w4_t(const SkinnyArgs& p, int group, hipStream_t stream) {
+  switch (group) {
+    case 128:
+      if (!p.scale_f32 && p.flags == QG_W4_ZEROS_PACKED) return launch_skinny_w4_g<SK_UINT4, F16A, 128>(p, stream);
+      return launch_skinny_w4_g<SK_W4, F16A, 128>(p, stream);
+    case 64: return launch_skinny_w4_g<SK_W4, F16A, 64>(p, stream);
+    default: return launch_skinny_w4_g<SK_W4, F16A, 32>(p, stream);
+  }
+}
+
 }  // namespace
+
+bool skinny_w4_applies(const W4Args& p) {
+  if (p.M < 1 || p.M > kSkinnyMaxRows || (p.flags & QG_W4_LAYOUT_KN)) return false;
+  if (((reinterpret_cast<uintptr_t>(p.scales) | reinterpret_cast<uintptr_t>(p.zeros)) & 3) != 0) return false;
+  SkinnyArgs t{};
+  t.flags = p.flags;
+  t.ng = p.ng;
+  t.zw = p.zw;
+  t.scale_f32 = p.scale_f32;
+  // one column tile next to the rings of 16 rows (8 waves x 2 chunks x 5 KB)
+  return 80 * 1024 + skinny_par_bytes(t, 16) <= kMaxLds;
+}
+
+hipError_t launch_skinny_w4(const W4Args& p, hipStream_t stream) {
+  if (!skinny_w4_applies(p)) return hipErrorInvalidValue;
+  SkinnyArgs t{};
+  t.a = p.a;
+  t.a_sm = p.a_sm;
+  t.w = p.w;
+  t.w_sn = p.K / 2;
+  t.M = p.M;
+  t.N = p.N;
+  t.K = p.K;
+  t.flags = p.flags;
+  t.ng = p.ng;
+  t.zw = p.zw;
+  t.scales = p.scales;
+  t.scale_f32 = p.scale_f32;
+  t.zeros = p.zeros;
+  t.bias = p.bias;
+  t.bias_dtype = p.bias_dtype;
+  t.out = p.out;
+  t.out_dtype = p.out_dtype;
+  return p.a_f16 ? launch_skinny_w4_t<true>(t, p.group, stream) : launch_skinny_w4_t<false>(t, p.group, stream);
+}
 
 hipError_t launch_skinny_fp8(const SkinnyArgs& p, bool f16a, bool e5, hipStream_t stream) {
   if (p.M < 1 || p.M > kSkinnyMaxRows || p.K % 16 != 0 || p.K < 16) return hipErrorInvalidValue;

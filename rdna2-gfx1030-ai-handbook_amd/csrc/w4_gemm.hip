@@ -335,7 +335,8 @@ __global__ __launch_bounds__(64 * WAVES) void k_w4_skinny(W4Args p) {
 }
 
 // ------------------------------------------------------------- decode kernel
-// M <= 16 (token decode), the HBM-bound shape. One workgroup of WAVES waves
+// M <= 16 (token decode), the HBM-bound shape: the kn layout, and uint4 storage
+// where it beats the streaming kernel (uint4_decode_applies). One workgroup of WAVES waves
 // per 16*CT output columns; wave w owns a contiguous range of 128-wide K
 // chunks (at most CH, 4 or 8). At the start each wave copies its
 // activation slice [rows, 128 * chunks] into its own LDS region (one 16-byte
@@ -486,13 +487,6 @@ __global__ __launch_bounds__(64 * WAVES) void k_w4_decode(W4Args p) {
       if constexpr (!KN && G == 128) {
         const i32x4 v = load_at<i32x4>(p.w, woff(n, kw0 + 4 * q));
         static_for<0, 4>([&](auto j) { ch[cl].w[t][j] = static_cast<uint32_t>(v[int(j)]); });
-      } else if constexpr (!KN && G == 64) {
-        const uint2 v0 = load_at<uint2>(p.w, woff(n, kw0 + 2 * q));
-        const uint2 v1 = load_at<uint2>(p.w, woff(n, min(kw0 + 8 + 2 * q, KW - 2)));
-        ch[cl].w[t][0] = v0.x;
-        ch[cl].w[t][1] = v0.y;
-        ch[cl].w[t][2] = v1.x;
-        ch[cl].w[t][3] = v1.y;
       } else {
         static_for<0, 4>([&](auto j) {
           ch[cl].w[t][j] = load_at<uint32_t>(p.w, woff(n, min(kw0 + word_of<G, KN>(q, j), KW - 1)));
@@ -937,43 +931,54 @@ hipError_t launch_decode_t(const W4Args& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// kn layout (consecutive columns are consecutive words).
 template <int RP, int CT, bool F16A>
-hipError_t launch_decode_g(const W4Args& p, hipStream_t stream) {
-  const bool kn = p.flags & QG_W4_LAYOUT_KN;
+hipError_t launch_decode_kn(const W4Args& p, hipStream_t stream) {
   switch (p.group) {
-    case 128: {
-      const int cpw = ceil_div(ceil_div(p.K, 128), 8);
-      if (!kn && !p.scale_f32 && p.flags == QG_W4_ZEROS_PACKED && p.ng % 4 == 0 && cpw == kDecodeChunks)
-        return launch_decode_t<RP, CT, 128, false, F16A, true>(p, stream);
-      return kn ? launch_decode_t<RP, CT, 128, true, F16A, false>(p, stream)
-                : launch_decode_t<RP, CT, 128, false, F16A, false>(p, stream);
-    }
-    case 64:
-      return kn ? launch_decode_t<RP, 2, 64, true, F16A, false>(p, stream)
-                : launch_decode_t<RP, 2, 64, false, F16A, false>(p, stream);
+    case 128: return launch_decode_t<RP, CT, 128, true, F16A, false>(p, stream);
+    case 64: return launch_decode_t<RP, 2, 64, true, F16A, false>(p, stream);
     default:  // group 32: one column tile per wave past one row (4 scale / zero words per chunk)
-      return kn ? launch_decode_t<RP, (RP > 1 ? 1 : 2), 32, true, F16A, false>(p, stream)
-                : launch_decode_t<RP, (RP > 1 ? 1 : 2), 32, false, F16A, false>(p, stream);
+      return launch_decode_t<RP, (RP > 1 ? 1 : 2), 32, true, F16A, false>(p, stream);
   }
+}
+
+// uint4 storage whose 8 waves take exactly 4 chunks each (K 3585 .. 4096): the
+// decode kernel with all loads up front, against the streaming kernel of
+// skinny_gemm.hip, at K 4096 (us, both rotated weight copies, one box):
+//   N      M 4            M 8             M 16
+//   14336  9.3 / 10.1     10.8 / 10.8     11.1 / 12.1
+//   8192   5.8 / 6.4      8.9 / 6.9       9.2 / 7.9
+//   4096   5.2 / 4.8      8.7 / 5.3       9.0 / 6.0
+// and everywhere else the streaming kernel (group 64: M 1 / 16, N 14336, 24.1 /
+// 27.9 -> 12.1 / 17.1; group 32 45 / 52 -> 15 / 21; K 14336, N 4096, M 16
+// uint4 43.6 -> 14.1, from 64 workgroups of k_w4_skinny with two chunks in flight).
+bool uint4_decode_applies(const W4Args& p) {
+  return p.group == 128 && !p.scale_f32 && p.flags == QG_W4_ZEROS_PACKED && p.ng % 4 == 0 &&
+         ceil_div(ceil_div(p.K, 128), 8) == kDecodeChunks && p.M > 1 && p.N >= (p.M <= 4 ? 8192 : 12288);
 }
 
 template <bool F16A>
 hipError_t launch_skinny(const W4Args& p, hipStream_t stream) {
   const int C = ceil_div(p.K, 128);
-  if (p.M <= 16 && ceil_div(C, 8) <= kDecodeChunks) {
-    // column tiles of 16 per workgroup, all sharing each activation fragment:
-    // two for 1-4 rows (cfg2, 448 workgroups: 2-4 rows 9.5-9.7 us against
-    // 10.0-10.1 us with four), four for 5-16 rows (11.2-11.4 us against 12.9 us
-    // with two)
-    if (p.M == 1) {
-      if (gemv1_applies(p)) {
-        hipLaunchKernelGGL(k_w4_gemv1, dim3(ceil_div(p.N, 32)), dim3(512), 0, stream, p);
-        return hipGetLastError();
-      }
-      return launch_decode_g<1, 2, F16A>(p, stream);
+  const bool kn = p.flags & QG_W4_LAYOUT_KN;
+  if (p.M <= 16 && !kn) {
+    if (gemv1_applies(p)) {
+      hipLaunchKernelGGL(k_w4_gemv1, dim3(ceil_div(p.N, 32)), dim3(512), 0, stream, p);
+      return hipGetLastError();
     }
-    if (p.M <= 4) return launch_decode_g<4, 2, F16A>(p, stream);
-    return launch_decode_g<16, 4, F16A>(p, stream);
+    if (uint4_decode_applies(p)) {
+      // column tiles of 16 per workgroup, all sharing each activation fragment:
+      // two for 2-4 rows (cfg2, 448 workgroups: 9.5-9.7 us against 10.0-10.1 us
+      // with four), four for 5-16 rows (11.2-11.4 us against 12.9 us with two)
+      if (p.M <= 4) return launch_decode_t<4, 2, 128, false, F16A, true>(p, stream);
+      return launch_decode_t<16, 4, 128, false, F16A, true>(p, stream);
+    }
+    if (skinny_w4_applies(p)) return launch_skinny_w4(p, stream);
+  }
+  if (p.M <= 16 && kn && ceil_div(C, 8) <= kDecodeChunks) {
+    if (p.M == 1) return launch_decode_kn<1, 2, F16A>(p, stream);
+    if (p.M <= 4) return launch_decode_kn<4, 2, F16A>(p, stream);
+    return launch_decode_kn<16, 4, F16A>(p, stream);
   }
   if (p.M <= 16) return launch_skinny_g<1, 4, F16A>(p, stream);
   if (p.M <= 32) return launch_skinny_g<2, 1, F16A>(p, stream);

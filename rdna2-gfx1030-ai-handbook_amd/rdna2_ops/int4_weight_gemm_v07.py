@@ -289,6 +289,15 @@ def _gemv1_applies(a, p):
             and p.scales.data_ptr() % 4 == 0 and p.zeros.data_ptr() % 4 == 0)
 
 
+def _skinny_par_bytes(p, cols):
+    """LDS bytes of the group parameters of ``cols`` columns in the few-row
+    kernel (skinny_par_bytes in csrc/skinny_gemm.hip)."""
+    ng = p.k // p.group_size
+    s = cols * ((ng if p.scales.dtype == torch.float32 else ng // 2 + 1) | 1)
+    z = cols * (((ng + 7) // 8 if p.zeros_packed else ng) | 1)
+    return 4 * (-(-s // 64) * 64 + -(-z // 64) * 64)
+
+
 def w4a16_gemm(a, p, bias=None, *, out_dtype=None):
     """The fused W4A16 kernel: out = a @ dequant(p)^T (+ bias), fp32
     accumulation, one rounding to out_dtype (default: a's dtype)."""
@@ -340,8 +349,8 @@ def int4_linear_a16(a, p, *, bias=None, method="dequant", prepared=None, tile=(6
     if return_kernel:
         # the C ABI's choice: past 64 rows the dequant formulation from the
         # group's tile threshold (K a multiple of 64), else the tiled MFMA kernel
-        # (K a multiple of 128); the decode kernels for up to 16 rows and K <=
-        # 4096; else skinny
+        # (K a multiple of 128); up to 16 rows the one-row, decode and
+        # streaming kernels; else skinny
         m = a.shape[0]
         if _lib.library().qg_w4a16_gemm_workspace_bytes(m, p.n, p.k, p.group_size, p.flags) > 0:
             # prefill grid at or past the group's threshold of 256 x 192 tiles
@@ -360,11 +369,32 @@ def int4_linear_a16(a, p, *, bias=None, method="dequant", prepared=None, tile=(6
             hint = "k_wd_gemmILi{}ELi{}ELb{}ELb{}ELi2ELi4ELi128ELi{}E".format(
                 fmt, p.group_size, int(bool(p.flags & _lib.W4_LAYOUT_KN)), int(a.dtype == torch.float16), tbn)
             return out, _lib.kernel_metadata("w4a16_tiled_mfma", (128, tbn, 128), hint)
-        if m <= 16 and -(-p.k // 128) <= 32:
+        kn, f16 = bool(p.flags & _lib.W4_LAYOUT_KN), int(a.dtype == torch.float16)
+        if m <= 16 and not kn:
             if _gemv1_applies(a, p):
                 return out, _lib.kernel_metadata("w4a16_gemv1", (1, 32, 512), "k_w4_gemv1")
+            uint4 = p.flags == _lib.W4_ZEROS_PACKED and p.group_size == 128 and p.scales.dtype == torch.bfloat16
+            ng = p.k // p.group_size
+            if (uint4 and ng % 4 == 0 and -(-(-(-p.k // 128)) // 8) == 4 and m > 1
+                    and p.n >= (8192 if m <= 4 else 12288)):
+                rp, ct = (4, 2) if m <= 4 else (16, 4)
+                return out, _lib.kernel_metadata("w4a16_decode", (rp, 16 * ct, 128),
+                                                 "k_w4_decodeILi{}ELi{}ELi128E".format(rp, ct))
+            if _skinny_par_bytes(p, 16) <= 80 * 1024:
+                rp = 4 if m <= 4 else 8 if m <= 8 else 16
+                if p.k <= 512:
+                    ct = 2 if rp == 4 else {128: 4, 64: 2, 32: 1}[p.group_size]
+                else:
+                    ct = _lib.skinny_tiles(p.n, rp // 4, 1, (1, 2, 4) if rp == 16 and p.group_size != 32 else (1, 2))
+                while ct > 1 and 4096 * rp + 16384 * ct + _skinny_par_bytes(p, 16 * ct) > 160 * 1024:
+                    ct //= 2
+                return out, _lib.kernel_metadata(
+                    "w4a16_decode", (rp, 16 * ct, 128),
+                    "k_skinny_gemmINS0_9SkinnyCfgILi{}ELb{}ELi{}ELi{}ELi2ELi{}E".format(
+                        4 if uint4 else 3, f16, rp, ct, p.group_size))
+        if m <= 16 and kn and -(-p.k // 128) <= 32:
             rp = 1 if m == 1 else 4 if m <= 4 else 16
-            # column tiles of 16 per workgroup, as launch_decode_g picks them
+            # column tiles of 16 per workgroup, as launch_decode_kn picks them
             ct = (4 if rp == 16 else 2) if p.group_size == 128 else 2 if p.group_size == 64 else (1 if rp > 1 else 2)
             return out, _lib.kernel_metadata("w4a16_decode", (rp, 16 * ct, 128),
                                              "k_w4_decodeILi{}ELi{}ELi{}E".format(rp, ct, p.group_size))

@@ -6,7 +6,9 @@ import torch
 
 from conftest import case
 from oracle import fp8 as o8
+from oracle import int4 as o4
 from test_fp8_gpu import check, codes_tensor
+from test_w4_gpu import act_values, check_product
 
 pytestmark = pytest.mark.gpu
 
@@ -67,3 +69,67 @@ def test_fp8_values_past_k(cuda):
     w = codes_tensor(store, False, cuda)[:, :k]
     y = fp8_weight_gemm(torch.ones(3, k, dtype=torch.bfloat16, device=cuda), w, method="fused_dot2")
     assert torch.equal(y.float().cpu(), torch.full((3, n), float(k)))
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 1, 640), (4, 17, 1088), (5, 33, 2176), (8, 4100, 768), (9, 47, 4160), (16, 16, 2048), (16, 8208, 1024),
+    (16, 14337, 640), (3, 96, 512),
+])
+@pytest.mark.parametrize("g", o4.GROUPS)
+@pytest.mark.parametrize("sym,order,adtype", [(True, "low", torch.float16), (False, "high", torch.bfloat16)])
+def test_int4_shapes(cuda, m, n, k, g, sym, order, adtype):
+    """Signed INT4 (nk): row counts, one to four column tiles, an odd number
+    of groups and a last chunk of fewer groups, both nibble orders, bias."""
+    from rdna2_ops import int4_weight_gemm_v07 as w4
+    k = k // g * g
+    case(f"skinny int4 {m}x{n}x{k} g{g} sym={sym} {order} {adtype}")
+    gen = torch.Generator().manual_seed(m + n + k + g)
+    w = torch.randn(n, k, generator=gen) * 0.02
+    a = torch.randn(m, k + 8, generator=gen).to(adtype)[:, :k]
+    b = (torch.randn(n, generator=gen) * 0.1).to(adtype)
+    p = w4.pack_int4(w.to(cuda), group_size=g, symmetric=sym, order=order)
+    cen = w4.unpack_int4(p, dtype=torch.int8).cpu().numpy().astype(np.int32)
+    s = p.scales.cpu().numpy()
+    av = act_values(a)
+    y64 = o4.w4a16_linear(av, cen, s, g, act_values(b))
+    absmag = o4.w4a16_linear(np.abs(av), np.ones_like(cen), s, g)
+    y = w4.int4_linear_a16(a.to(cuda), p, bias=b.to(cuda), method="dot2")
+    check_product(y, y64, absmag, adtype, f"skinny int4 {m}x{n}x{k} g{g}")
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 50, 1152), (2, 33, 14336), (6, 4097, 1152), (16, 40, 14336), (16, 12300, 3200)])
+@pytest.mark.parametrize("adtype", [torch.float16, torch.bfloat16])
+def test_uint4_shapes(cuda, m, n, k, adtype):
+    """uint4 storage with bf16 scales: an odd number of groups (a column's
+    scales start in the upper half of a word) and K past the decode kernels'."""
+    from rdna2_ops import int4_weight_gemm_v07 as w4
+    case(f"skinny uint4 {m}x{n}x{k} {adtype}")
+    gen = torch.Generator().manual_seed(m + n + k)
+    w = torch.randn(n, k, generator=gen) * 0.02
+    a = torch.randn(m, k, generator=gen).to(adtype)
+    p = w4.pack_uint4(w.to(cuda), group_size=128)
+    cen = w4.unpack_int4(p, dtype=torch.int8).cpu().numpy().astype(np.int32)
+    s = p.scales.float().cpu().numpy()
+    av = act_values(a)
+    y64 = o4.w4a16_linear(av, cen, s, 128)
+    absmag = o4.w4a16_linear(np.abs(av), np.ones_like(cen), s, 128)
+    y = w4.int4_linear_a16(a.to(cuda), p, method="dot2")
+    check_product(y, y64, absmag, adtype, f"skinny uint4 {m}x{n}x{k}")
+
+
+def test_int4_parameters_past_lds(cuda):
+    """More groups than fit next to the rings (group 32, K 32768): the
+    kernel without LDS parameters."""
+    from rdna2_ops import int4_weight_gemm_v07 as w4
+    case("skinny int4 g32 k32768")
+    gen = torch.Generator().manual_seed(3)
+    n, k, g = 24, 32768, 32
+    w = torch.randn(n, k, generator=gen) * 0.02
+    a = torch.randn(3, k, generator=gen).to(torch.bfloat16)
+    p = w4.pack_int4(w.to(cuda), group_size=g)
+    cen = w4.unpack_int4(p, dtype=torch.int8).cpu().numpy().astype(np.int32)
+    av, s = act_values(a), p.scales.cpu().numpy()
+    y, md = w4.int4_linear_a16(a.to(cuda), p, method="dot2", return_kernel=True)
+    assert md["variant"] == "w4a16_skinny"
+    check_product(y, o4.w4a16_linear(av, cen, s, g), o4.w4a16_linear(np.abs(av), np.ones_like(cen), s, g),
+                  torch.bfloat16, "skinny int4 g32 k32768")
