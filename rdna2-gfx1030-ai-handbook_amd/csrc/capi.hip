@@ -30,9 +30,10 @@ constexpr int64_t kMaxOperandBytes = int64_t(1) << 31;
 constexpr int64_t kMoeMaxItems = 131072;
 
 // An operand of `rows` rows (row stride s_row, element stride s_k) can be read
-// in place by the GEMM kernel.
-inline bool canonical_rows(const void* p, int64_t s_row, int64_t s_k, int64_t rows, int64_t k) {
-  return s_k == 1 && (s_row % 16) == 0 && aligned16(p) && (k % kStageK) == 0 &&
+// in place by the GEMM kernel, which takes K in units of `whole`.
+inline bool canonical_rows(const void* p, int64_t s_row, int64_t s_k, int64_t rows, int64_t k,
+                           int64_t whole = kStageK) {
+  return s_k == 1 && (s_row % 16) == 0 && aligned16(p) && (k % whole) == 0 &&
          (rows - 1) * s_row + k < kMaxOperandBytes;
 }
 
@@ -40,7 +41,9 @@ inline bool float_dtype(int d) { return d == QG_F32 || d == QG_F16 || d == QG_BF
 
 struct I8Plan {
   bool pack_a, pack_b;
-  int64_t kp;
+  bool skinny;  // up to 16 rows: the streaming kernel of skinny_gemm.hip
+  int64_t kp;   // row length of packed operands
+  int64_t ks;   // K of the kernel: k, or kp where both operands are packed
   size_t a_bytes, b_bytes;
   size_t total() const { return a_bytes + b_bytes; }
 };
@@ -49,9 +52,13 @@ I8Plan plan_i8(const void* a, int64_t a_sm, int64_t a_sk, const void* b, int64_t
                int64_t b_sn, int64_t m, int64_t n, int64_t k) {
   I8Plan pl;
   pl.kp = round_up(k, kStageK);
+  pl.skinny = m <= qg::kSkinnyMaxRows && k > 0;
+  // the streaming kernel takes whole 16-byte chunks of a row, the tiled ones whole stages
+  const int64_t whole = pl.skinny ? 16 : kStageK;
+  pl.ks = k % whole == 0 ? k : pl.kp;
   // B = W^T: W [n, k] has row stride b_sn and element stride b_sk.
-  pl.pack_a = !canonical_rows(a, a_sm, a_sk, m, k);
-  pl.pack_b = !canonical_rows(b, b_sn, b_sk, n, k);
+  pl.pack_a = !canonical_rows(a, a_sm, a_sk, m, k, whole);
+  pl.pack_b = !canonical_rows(b, b_sn, b_sk, n, k, whole);
   pl.a_bytes = pl.pack_a ? static_cast<size_t>(round_up(m * pl.kp, 256)) : 0;
   pl.b_bytes = pl.pack_b ? static_cast<size_t>(round_up(n * pl.kp, 256)) : 0;
   return pl;
@@ -156,7 +163,7 @@ int int8_gemm_impl(const int8_t* a, int64_t a_sm, int64_t a_sk, const int8_t* b,
   qg::I8GemmArgs p{};
   p.M = static_cast<int>(m);
   p.N = static_cast<int>(n);
-  p.K = static_cast<int>(pl.kp);
+  p.K = static_cast<int>(pl.ks);
   char* ws = static_cast<char*>(workspace);
   if (pl.pack_a) {
     int8_t* pa = reinterpret_cast<int8_t*>(ws);
@@ -186,7 +193,7 @@ int int8_gemm_impl(const int8_t* a, int64_t a_sm, int64_t a_sk, const int8_t* b,
   p.out = out;
   p.out_dtype = out_dtype;
   p.epi = epilogue;
-  return qg::launch_i8_gemm(p, stream);
+  return pl.skinny ? qg::launch_skinny_i8(p, stream) : qg::launch_i8_gemm(p, stream);
 }
 
 }  // namespace
@@ -231,9 +238,9 @@ extern "C" int qg_int8_gemm_stages(const int8_t* a, const int8_t* w, int64_t m, 
 }
 
 namespace {
-// Workspace of the W8A8 linear: int8 activations [m, kp], fp32 steps [m], then
-// a packed copy of W when W is not canonical ([n, k] row-major, 16-byte rows,
-// k % 64 == 0).
+// Workspace of the W8A8 linear: int8 activations [m, kp] (zero past k), fp32
+// steps [m], then a packed copy of W when W is not canonical ([n, k] row-major,
+// 16-byte rows, k a multiple of the kernel's K unit).
 struct W8A8Plan {
   int64_t kp;
   size_t act_bytes, step_bytes;
@@ -311,7 +318,7 @@ int w8a8_linear_run(const void* x, int x_dtype, int64_t x_sm, int64_t m, int64_t
   p.residual_scalar = ex.residual_scale_numel == 1;
   p.M = static_cast<int>(m);
   p.N = static_cast<int>(n);
-  p.K = static_cast<int>(pl.kp);
+  p.K = static_cast<int>(pl.w.ks);
   p.a = xq;
   p.a_sm = pl.kp;
   if (pl.w.pack_b) {
@@ -332,7 +339,7 @@ int w8a8_linear_run(const void* x, int x_dtype, int64_t x_sm, int64_t m, int64_t
   p.out = out;
   p.out_dtype = out_dtype;
   p.epi = epilogue;
-  return qg::launch_i8_gemm(p, s);
+  return pl.w.skinny ? qg::launch_skinny_i8(p, s) : qg::launch_i8_gemm(p, s);
 }
 
 }  // namespace

@@ -224,6 +224,8 @@ struct SkinnyArgs {
   I8GemmArgs i8;         // int8: the epilogue's arguments (the fields above are the operands)
 };
 constexpr int kSkinnyMaxRows = 16;
+// int8 A and W; p.K a multiple of 16, every epilogue of launch_i8_gemm.
+hipError_t launch_skinny_i8(const I8GemmArgs& p, hipStream_t stream);
 hipError_t launch_skinny_fp8(const SkinnyArgs& p, bool f16a, bool e5, hipStream_t stream);
 // nk layout, M <= 16, group parameters that fit in LDS.
 bool skinny_w4_applies(const W4Args& p);

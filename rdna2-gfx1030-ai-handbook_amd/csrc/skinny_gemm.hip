@@ -496,4 +496,18 @@ hipError_t launch_skinny_fp8(const SkinnyArgs& p, bool f16a, bool e5, hipStream_
   return e5 ? launch_skinny_fp8_rows<SK_E5M2, false>(p, stream) : launch_skinny_fp8_rows<SK_E4M3, false>(p, stream);
 }
 
+hipError_t launch_skinny_i8(const I8GemmArgs& p, hipStream_t stream) {
+  if (p.M < 1 || p.M > kSkinnyMaxRows || p.K % 16 != 0 || p.K < 16) return hipErrorInvalidValue;
+  SkinnyArgs t{};
+  t.a = p.a;
+  t.a_sm = p.a_sm;
+  t.w = p.w;
+  t.w_sn = p.w_sn;
+  t.M = p.M;
+  t.N = p.N;
+  t.K = p.K;
+  t.i8 = p;
+  return p.M <= 8 ? launch_skinny_bytes<SK_I8, false, 8>(t, stream) : launch_skinny_bytes<SK_I8, false, 16>(t, stream);
+}
+
 }  // namespace qg

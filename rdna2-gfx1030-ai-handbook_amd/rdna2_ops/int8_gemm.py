@@ -134,12 +134,19 @@ def _launch(a, b, a_scale, b_scale, bias, *, tile, num_warps, num_stages, group_
     _lib.check(status, "qg_int8_gemm")
     if not return_kernel:
         return out
-    # the C ABI's choice: >= 192 tiles of 256 x 192 take the persistent 8-wave
-    # ping-pong kernel, smaller grids the 4-wave 128 x 128 one (K stage 128)
-    big = (-(-m // 256)) * (-(-n // 192)) >= 192
-    tile_used = (256, 192, 128) if big else (128, 128, 128)
-    meta = _lib.kernel_metadata("int8_mfma_32x32x32_pingpong" if big else "int8_mfma_32x32x32", tile_used,
-                                "k_i8_gemm_ppINS0_5I8GeoILi256ELi192E" if big else "k_i8_gemmINS0_5I8GeoILi128ELi128E")
+    # the C ABI's choice: up to 16 rows the streaming kernel; >= 192 tiles of
+    # 256 x 192 the persistent 8-wave ping-pong kernel, smaller grids the
+    # 4-wave 128 x 128 one (K stage 128)
+    if m <= 16 and k > 0:
+        rows = 8 if m <= 8 else 16
+        ct = _lib.skinny_tiles(n, rows // 8, 2)
+        meta = _lib.kernel_metadata("int8_mfma_16x16x64_skinny", (rows, 16 * ct, 128),
+                                    "k_skinny_gemmINS0_9SkinnyCfgILi0ELb0ELi{}ELi{}E".format(rows, ct))
+    elif (-(-m // 256)) * (-(-n // 192)) >= 192:
+        meta = _lib.kernel_metadata("int8_mfma_32x32x32_pingpong", (256, 192, 128),
+                                    "k_i8_gemm_ppINS0_5I8GeoILi256ELi192E")
+    else:
+        meta = _lib.kernel_metadata("int8_mfma_32x32x32", (128, 128, 128), "k_i8_gemmINS0_5I8GeoILi128ELi128E")
     meta.update(packed_operands=ws_bytes > 0, requested_tile=list(tile), epilogue_flags=flags,
                 requested_wrapped=bool(wrapped), requested_partial_dot=bool(partial_dot))
     return out, meta

@@ -7,6 +7,7 @@ import torch
 from conftest import case
 from oracle import fp8 as o8
 from oracle import int4 as o4
+from oracle import int8 as oi
 from test_fp8_gpu import check, codes_tensor
 from test_w4_gpu import act_values, check_product
 
@@ -133,3 +134,60 @@ def test_int4_parameters_past_lds(cuda):
     assert md["variant"] == "w4a16_skinny"
     check_product(y, o4.w4a16_linear(av, cen, s, g), o4.w4a16_linear(np.abs(av), np.ones_like(cen), s, g),
                   torch.bfloat16, "skinny int4 g32 k32768")
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 1, 16), (2, 17, 144), (8, 33, 1040), (9, 48, 2064), (16, 4097, 256), (16, 768, 3072), (3, 12304, 160),
+    (16, 20, 8), (11, 31, 257), (4, 40, 131056),
+])
+def test_int8_shapes(cuda, m, n, k):
+    """int32 sums bit-exact (tails, packed operands, strided rows), and every
+    epilogue against the oracle: orders F, FMA and eager, GELU within the
+    activation's own bound elsewhere; scalar and per-column scales."""
+    from rdna2_ops.int8_gemm import int8_gemm_dequant, int8_matmul
+    case(f"skinny int8 {m}x{n}x{k}")
+    g = torch.Generator().manual_seed(m * 31 + n * 7 + k)
+    a = torch.randint(-128, 128, (m, k + 16), generator=g, dtype=torch.int8)
+    w = torch.randint(-128, 128, (n, k), generator=g, dtype=torch.int8)
+    sa, sb = torch.rand(m, generator=g) * 0.02 + 0.001, torch.rand(n, generator=g) * 0.02 + 0.001
+    bias = torch.randn(n, generator=g)
+    acc = oi.int8_matmul(a[:, :k].numpy(), np.ascontiguousarray(w.numpy().T))
+    ag, wg, sag, sbg, bg = a.to(cuda)[:, :k], w.to(cuda), sa.to(cuda), sb.to(cuda), bias.to(cuda)
+    assert np.array_equal(int8_matmul(ag, wg.T).cpu().numpy(), acc)
+    for out, dt in (("f32", torch.float32), ("f16", torch.float16), ("bf16", torch.bfloat16)):
+        def same(got, ref):
+            return np.array_equal(got.cpu().float().numpy(), np.asarray(oi.round_to(ref, out), np.float32))
+        kw = dict(out_dtype=dt)
+        assert same(int8_gemm_dequant(ag, wg.T, sag, sbg, bg, **kw),
+                    oi.epilogue_f(acc, sa.numpy(), sb.numpy(), bias.numpy(), out=out))
+        assert same(int8_gemm_dequant(ag, wg.T, sag, sbg[:1].contiguous(), None, **kw),
+                    oi.epilogue_f(acc, sa.numpy(), np.full(n, sb[0].item(), np.float32), None, out=out))
+        assert same(int8_gemm_dequant(ag, wg.T, sag, sbg, bg, epilogue_order="eager", **kw),
+                    oi.epilogue_e(acc, sa.numpy(), sb.numpy(), bias.numpy(), out=out))
+    y, md = int8_gemm_dequant(ag, wg.T, sag, sbg, bg, rounding="fused", return_kernel=True)
+    assert md["variant"] == "int8_mfma_16x16x64_skinny" and md["vgpr"] is not None
+    scale = (sa.numpy()[:, None] * sb.numpy()[None, :]).astype(np.float32)
+    ref = (acc.astype(np.float32).astype(np.float64) * scale + bias.numpy()).astype(np.float32)  # one rounding
+    assert np.array_equal(y.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("m,k", [(2, 3072), (16, 1040), (5, 200)])
+def test_int8_linear_same_as_wider_batch(cuda, m, k):
+    """The W8A8 linear of a few rows equals the same rows of a wider batch
+    (the tiled kernels) bit for bit: quantizer, GELU, residual and scale."""
+    from rdna2_ops.int8_gemm import w8a8_linear
+    case(f"skinny w8a8 {m}x{k}")
+    g = torch.Generator().manual_seed(k)
+    n = 150
+    x = torch.randn(40, k, generator=g).to(torch.float16).to(cuda)
+    w = torch.randint(-127, 128, (n, k), generator=g, dtype=torch.int8).to(cuda)
+    ws, b = (torch.rand(n, generator=g) * 0.01).to(cuda), torch.randn(n, generator=g).to(cuda)
+    res = torch.randn(40, n, generator=g).to(torch.bfloat16).to(cuda)
+    rs = torch.rand(n, generator=g).to(cuda)
+    for kw in (dict(), dict(activation="gelu_tanh"), dict(residual=True), dict(activation="gelu_tanh", residual=True)):
+        def call(rows):
+            extra = dict(kw)
+            if extra.pop("residual", False):
+                extra.update(residual=res[:rows], residual_scale=rs)
+            return w8a8_linear(x[:rows], w, ws, b, **extra)
+        assert torch.equal(call(m).view(torch.int16), call(40)[:m].view(torch.int16)), kw
