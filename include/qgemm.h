@@ -270,7 +270,11 @@ int qg_w4_unpack(const int32_t* data, int64_t n, int64_t k, int group_size,
  * workspace, (q - z) * s in fp32 rounded to the activation dtype, then a
  * 2-byte MFMA GEMM with fp32 accumulation runs on it; the workspace is then
  * 2 * n * k bytes (16-byte aligned), reported by
- * qg_w4a16_gemm_workspace_bytes (0 on the other shapes), and required.
+ * qg_w4a16_gemm_workspace_bytes, and required. nk weights with K >= 1024 and
+ * up to 2048 rows keep the exact group sums instead where that is faster; K
+ * may then be split over workgroups, with fp32 partial tiles in the workspace
+ * that qg_w4a16_gemm_workspace_bytes reports (without it the call runs
+ * unsplit). 0 on the other shapes.
  * a: [m, k] QG_F16 or QG_BF16, unit K stride, row stride a_sm (a multiple of 8
  * elements, 16-byte aligned base); w: 16-byte aligned; out: [m, n] contiguous
  * QG_F16 / QG_BF16 / QG_F32; bias NULL or [n] of bias_dtype; m * n < 2^31. */
@@ -475,6 +479,17 @@ int qg_mfma_clock(int mode, int iters, uint32_t* out, void* stream);
 int qg_int8_gemm_stages(const int8_t* a, const int8_t* w, int64_t m, int64_t n, int64_t k, const float* a_scale,
                         const float* w_scale, const void* bias_f16, void* out_f16, uint32_t* stamps,
                         size_t stamp_words, void* stream);
+
+/* ---------------------------------------------------------------------------
+ * Kernel choice past 16 rows (for the operators' kernel metadata; no
+ * counterpart in the reference), for canonical operands with the workspace
+ * that the call's query reports: splits << 16 | tile rows of the multi-stage
+ * kernel (tiles of 128 columns), QG_CHOICE_DEQUANT or QG_CHOICE_PINGPONG, or 0
+ * for the kernels of the shorter or larger grids.
+ * ------------------------------------------------------------------------- */
+enum qg_choice_format { QG_CHOICE_W4A16 = 0, QG_CHOICE_FP8 = 1, QG_CHOICE_INT8 = 2 };
+enum qg_choice { QG_CHOICE_DEQUANT = 1, QG_CHOICE_PINGPONG = 2 };
+int qg_row_kernel_choice(int format, int group_size, int flags, int64_t m, int64_t n, int64_t k);
 
 #ifdef __cplusplus
 }

@@ -42,11 +42,22 @@ inline bool float_dtype(int d) { return d == QG_F32 || d == QG_F16 || d == QG_BF
 struct I8Plan {
   bool pack_a, pack_b;
   bool skinny;  // up to 16 rows: the streaming kernel of skinny_gemm.hip
+  qg::MidPlan mid;  // splits > 1: K split over workgroups of mid_gemm.hip, given the workspace
   int64_t kp;   // row length of packed operands
   int64_t ks;   // K of the kernel: k, or kp where both operands are packed
   size_t a_bytes, b_bytes;
-  size_t total() const { return a_bytes + b_bytes; }
+  size_t partial_bytes;
+  size_t packed() const { return a_bytes + b_bytes; }
+  size_t total() const { return a_bytes + b_bytes + partial_bytes; }
 };
+
+// Model time (us) of the tiled INT8 kernel on 128 x 128 tiles: rounds of 256,
+// 0.56 us per stage (N 3072, K 3072: 16.7 to 17.6 us for M 32 to 512; K 12288:
+// 57 to 61 us, against 17.7 us for M 64 split 8 ways).
+double tiled_i8_us(int64_t m, int64_t n, int64_t k) {
+  const int64_t tiles = ((m + 127) / 128) * ((n + 127) / 128);
+  return 4.0 + (tiles + 255) / 256 * ((k + 127) / 128) * 0.56;
+}
 
 I8Plan plan_i8(const void* a, int64_t a_sm, int64_t a_sk, const void* b, int64_t b_sk,
                int64_t b_sn, int64_t m, int64_t n, int64_t k) {
@@ -61,6 +72,10 @@ I8Plan plan_i8(const void* a, int64_t a_sm, int64_t a_sk, const void* b, int64_t
   pl.pack_b = !canonical_rows(b, b_sn, b_sk, n, k, whole);
   pl.a_bytes = pl.pack_a ? static_cast<size_t>(round_up(m * pl.kp, 256)) : 0;
   pl.b_bytes = pl.pack_b ? static_cast<size_t>(round_up(n * pl.kp, 256)) : 0;
+  pl.mid = qg::plan_mid(qg::MID_I8, 128, m, n, k);
+  // a second launch costs the host about 4 us: it has to win clearly more
+  if (pl.mid.bm == 0 || pl.mid.splits == 1 || pl.mid.us + 10.0 > tiled_i8_us(m, n, k)) pl.mid = qg::MidPlan{0, 1, 0.0};
+  pl.partial_bytes = pl.mid.bm > 0 ? static_cast<size_t>(round_up(4 * pl.mid.splits * m * n, 256)) : 0;
   return pl;
 }
 
@@ -76,6 +91,27 @@ bool valid_gemm_shape(int64_t m, int64_t n, int64_t k, int64_t a_sm, int64_t a_s
   if (a_sm < 0 || a_sk < 0 || b_sk < 0 || b_sn < 0) return false;
   if (m * n > (int64_t(1) << 40)) return false;
   return true;
+}
+
+// The INT8 GEMM on prepared operands: p.K elements of both rows. `partial`:
+// null or the plan's partial tiles.
+hipError_t run_i8(const qg::I8GemmArgs& p, const I8Plan& pl, void* partial, hipStream_t stream) {
+  if (pl.skinny) return qg::launch_skinny_i8(p, stream);
+  if (pl.mid.bm > 0 && partial) {
+    qg::MidArgs t{};
+    t.op.a = p.a;
+    t.op.a_sm = p.a_sm;
+    t.op.w = p.w;
+    t.op.w_sn = p.w_sn;
+    t.op.M = p.M;
+    t.op.N = p.N;
+    t.op.K = p.K;
+    t.op.i8 = p;
+    t.splits = pl.mid.splits;
+    t.partial = partial;
+    return qg::launch_mid_i8(t, stream);
+  }
+  return qg::launch_i8_gemm(p, stream);
 }
 
 }  // namespace
@@ -156,8 +192,10 @@ int int8_gemm_impl(const int8_t* a, int64_t a_sm, int64_t a_sk, const int8_t* b,
   if (m == 0 || n == 0) return hipSuccess;
   if (!out || (k > 0 && (!a || !b))) return hipErrorInvalidValue;
   const I8Plan pl = plan_i8(a, a_sm, a_sk, b, b_sk, b_sn, m, n, k);
-  if (pl.total() > 0 && (!workspace || workspace_bytes < pl.total() || !aligned16(workspace)))
+  if (pl.packed() > 0 && (!workspace || workspace_bytes < pl.packed() || !aligned16(workspace)))
     return hipErrorInvalidValue;
+  // a call without room for the partial tiles runs unsplit
+  const bool split = pl.partial_bytes > 0 && workspace && workspace_bytes >= pl.total() && aligned16(workspace);
   if (m * pl.kp >= kMaxOperandBytes || n * pl.kp >= kMaxOperandBytes) return hipErrorInvalidValue;
 
   qg::I8GemmArgs p{};
@@ -193,7 +231,7 @@ int int8_gemm_impl(const int8_t* a, int64_t a_sm, int64_t a_sk, const int8_t* b,
   p.out = out;
   p.out_dtype = out_dtype;
   p.epi = epilogue;
-  return pl.skinny ? qg::launch_skinny_i8(p, stream) : qg::launch_i8_gemm(p, stream);
+  return run_i8(p, pl, split ? ws + pl.packed() : nullptr, stream);
 }
 
 }  // namespace
@@ -245,7 +283,8 @@ struct W8A8Plan {
   int64_t kp;
   size_t act_bytes, step_bytes;
   I8Plan w;
-  size_t total() const { return act_bytes + step_bytes + w.b_bytes; }
+  size_t packed() const { return act_bytes + step_bytes + w.b_bytes; }
+  size_t total() const { return packed() + w.partial_bytes; }
 };
 W8A8Plan plan_w8a8(const void* w, int64_t w_sn, int64_t m, int64_t n, int64_t k) {
   W8A8Plan pl;
@@ -301,7 +340,8 @@ int w8a8_linear_run(const void* x, int x_dtype, int64_t x_sm, int64_t m, int64_t
   if (m == 0 || n == 0) return hipSuccess;
   if (!out || (k > 0 && (!x || !w))) return hipErrorInvalidValue;
   const W8A8Plan pl = plan_w8a8(w, w_sn, m, n, k);
-  if (!ws || capacity < pl.total() || !aligned16(ws)) return hipErrorInvalidValue;
+  if (!ws || capacity < pl.packed() || !aligned16(ws)) return hipErrorInvalidValue;
+  const bool split = pl.w.partial_bytes > 0 && capacity >= pl.total();
   if (m * pl.kp >= kMaxOperandBytes || n * pl.kp >= kMaxOperandBytes) return hipErrorInvalidValue;
   int8_t* xq = reinterpret_cast<int8_t*>(ws);
   float* xs = reinterpret_cast<float*>(ws + pl.act_bytes);
@@ -339,7 +379,7 @@ int w8a8_linear_run(const void* x, int x_dtype, int64_t x_sm, int64_t m, int64_t
   p.out = out;
   p.out_dtype = out_dtype;
   p.epi = epilogue;
-  return pl.w.skinny ? qg::launch_skinny_i8(p, s) : qg::launch_i8_gemm(p, s);
+  return run_i8(p, pl.w, split ? ws + pl.packed() : nullptr, s);
 }
 
 }  // namespace
@@ -424,7 +464,7 @@ extern "C" int qg_w8a8_linear_noalloc(const void* x, int x_dtype, int64_t x_sm, 
   // argument errors before any HIP call (the workspace check needs the plan)
   if (m < 0 || n < 0 || k < 0 || k > kMaxK || w_sn < 0) return hipErrorInvalidValue;
   if (m == 0 || n == 0) return hipSuccess;
-  if (plan_w8a8(w, w_sn, m, n, k).total() > QG_W8A8_NOALLOC_SCRATCH_BYTES) return hipErrorInvalidValue;
+  if (plan_w8a8(w, w_sn, m, n, k).packed() > QG_W8A8_NOALLOC_SCRATCH_BYTES) return hipErrorInvalidValue;
   // the scratch of the device the stream runs on, which must be the current one
   hipStream_t s = static_cast<hipStream_t>(stream);
   int device = -1;
@@ -531,12 +571,56 @@ size_t w4_prefill_bytes(int64_t m, int64_t n, int64_t k, int group_size) {
   return static_cast<size_t>(round_up(2 * n * k, 256));
 }
 
+// Model time (us) of a ping-pong GEMM on 2-byte activations: rounds of 256
+// tiles of 256 x 192, 0.8 us per 64-element stage (M 2048, N = K = 3072, 128
+// tiles of fp8: 69 us with the 128-row tiles of k_wd_gemm, 45 us this way).
+double pingpong_us(int64_t m, int64_t n, int64_t k) {
+  const int64_t tiles = ((m + 255) / 256) * ((n + 191) / 192);
+  return 5.0 + (tiles + 255) / 256 * ((k + 63) / 64) * 0.8;
+}
+
+// Model time (us) of k_w4_skinny (17 to 64 rows): workgroups of 16 columns,
+// rounds of 256, by group size and row tile (N 1024 to 12288, K 3072 to 12288).
+double skinny_w4_us(int64_t m, int64_t n, int64_t k, int group_size) {
+  const double stage = group_size == 128 ? (m <= 32 ? 0.33 : 0.56) : group_size == 64 ? (m <= 32 ? 0.41 : 0.64)
+                                                                                      : (m <= 32 ? 0.58 : 0.80);
+  return 1.5 + ((n + 15) / 16 + 255) / 256 * ((k + 127) / 128) * stage;
+}
+
+// The kernel of a W4A16 call past 16 rows in the nk layout with K >= 1024:
+// mid_gemm where its model beats, by 10 %, the kernel that served the call
+// before it: k_w4_skinny up to 64 rows, the dequant formulation where
+// w4_prefill_bytes asks for it (the unpack's bytes at 4.4 TB/s, then the
+// ping-pong GEMM), and in any case the tiled kernel (N 4096, K 4096, M 512,
+// group 128: 48 -> 36 us; group 64, M 333: 66 -> 44 us; N 3072, K 12288, M 512:
+// 129 -> 88 us). Calls that multiplied exact group sums still do: none moves to
+// the dequant formulation, which rounds the weights. kn layout and shorter K:
+// as w4_prefill_bytes says.
+struct W4Plan {
+  qg::MidPlan mid;       // bm > 0: mid_gemm
+  size_t dequant_bytes;  // > 0: dequant + ping-pong
+  size_t total(int64_t m, int64_t n) const {
+    if (mid.bm > 0) return mid.splits > 1 ? static_cast<size_t>(round_up(4 * mid.splits * m * n, 256)) : 0;
+    return dequant_bytes;
+  }
+};
+W4Plan plan_w4(int64_t m, int64_t n, int64_t k, int group_size, int flags) {
+  W4Plan pl{qg::MidPlan{0, 1, 0.0}, w4_prefill_bytes(m, n, k, group_size)};
+  if ((flags & QG_W4_LAYOUT_KN) || m <= qg::kSkinnyMaxRows || k < qg::kMidMinK) return pl;
+  pl.mid = qg::plan_mid(qg::MID_W4, group_size, m, n, k);
+  double before_us = 1.0e9;
+  if (m <= kW4TiledMinRows) before_us = skinny_w4_us(m, n, k, group_size);
+  else if (pl.dequant_bytes > 0) before_us = 2.5 + n * k * 2.5 / 4.4e6 + pingpong_us(m, n, k);
+  if (pl.mid.us > 0.9 * before_us) pl.mid.bm = 0;
+  return pl;
+}
+
 }  // namespace
 
 extern "C" size_t qg_w4a16_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k, int group_size,
                                                 int flags) {
   if (!valid_w4_shape(n, k, group_size, flags) || m < 0 || m > kIntMax) return 0;
-  return w4_prefill_bytes(m, n, k, group_size);
+  return plan_w4(m, n, k, group_size, flags).total(m, n);
 }
 
 extern "C" int qg_w4a8_gemm(const int8_t* a, int64_t a_sm, int64_t m, int64_t k, const int32_t* w, int64_t n,
@@ -620,12 +704,21 @@ extern "C" int qg_w4a16_gemm(const void* a, int a_dtype, int64_t a_sm, int64_t m
   p.bias_dtype = bias_dtype;
   p.out = out;
   p.out_dtype = out_dtype;
-  // prefill grids past the group's tile threshold: dequantise W into the
-  // workspace, then the 2-byte ping-pong GEMM (out = acc + bias, one rounding)
-  const size_t need = w4_prefill_bytes(m, n, k, group_size);
-  if (need > 0) {
-    if (!workspace || workspace_bytes < need || !aligned16(workspace)) return hipErrorInvalidValue;
-    hipStream_t s = static_cast<hipStream_t>(stream);
+  W4Plan pl = plan_w4(m, n, k, group_size, flags);
+  const size_t need = pl.total(m, n);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (need > 0 && (!workspace || workspace_bytes < need || !aligned16(workspace))) {
+    // the dequant formulation needs its workspace; without room for the
+    // partial tiles K is not split (up to 64 rows k_w4_skinny is faster then)
+    if (pl.mid.bm == 0) return hipErrorInvalidValue;
+    pl.mid.splits = 1;
+    if (m <= kW4TiledMinRows || qg::mid_w4_lds(pl.mid.bm, group_size, k) > 160 * 1024) pl.mid.bm = 0;
+    if (pl.mid.bm == 0 && pl.dequant_bytes > 0) return hipErrorInvalidValue;
+  }
+  if (pl.mid.bm > 0) return qg::launch_mid_w4(p, pl.mid.bm, pl.mid.splits, workspace, s);
+  // dequantise W into the workspace, then the 2-byte ping-pong GEMM (out = acc
+  // + bias, one rounding)
+  if (pl.dequant_bytes > 0) {
     qg::W4Args u = p;
     u.out = workspace;
     u.out_dtype = a_dtype;
@@ -686,11 +779,14 @@ bool fp8_dtype(int d) { return d == QG_E4M3 || d == QG_E5M2; }
 struct Fp8Plan {
   bool pack_a, pack_w;
   bool skinny;    // up to 16 rows: the streaming kernel of skinny_gemm.hip
+  qg::MidPlan mid;  // bm > 0: the kernel of mid_gemm.hip (unless pingpong)
   bool pingpong;  // large grid: the ping-pong GEMM with fp8 W stages converted in registers
   int64_t kp;     // row length of packed operands
   int64_t ks;     // K of the kernel: k, or kp where both operands are packed
   size_t a_bytes, w_bytes;
-  size_t total() const { return a_bytes + w_bytes; }
+  size_t partial_bytes;  // of mid's splits (a call without this workspace runs unsplit)
+  size_t packed() const { return a_bytes + w_bytes; }
+  size_t total() const { return a_bytes + w_bytes + partial_bytes; }
 };
 
 Fp8Plan plan_fp8(const void* a, int64_t a_sm, int64_t a_sk, const void* w, int64_t w_sn, int64_t w_sk,
@@ -698,9 +794,20 @@ Fp8Plan plan_fp8(const void* a, int64_t a_sm, int64_t a_sk, const void* w, int64
   Fp8Plan pl;
   pl.kp = round_up(k, kStageK);
   pl.skinny = m <= qg::kSkinnyMaxRows && k > 0;
-  // the streaming kernel takes whole 16-byte chunks of a row, the tiled ones whole stages
-  const int64_t whole = pl.skinny ? 16 : kStageK;
+  pl.mid = qg::plan_mid(qg::MID_FP8, 128, m, n, k);
+  // >= 192 tiles of 256 x 192 (the INT8 kernel's large-grid rule), or where the
+  // model puts it before mid_gemm's tiles: the ping-pong GEMM, fp8 W converted
+  // exactly to A's 2-byte type in registers
+  const int64_t tiles = ((m + 255) / 256) * ((n + 191) / 192);
+  pl.pingpong = !pl.skinny && 2 * m * pl.kp < kMaxOperandBytes &&
+                (tiles >= 192 || (m > qg::kSkinnyMaxRows && k >= qg::kMidMinK &&
+                                  (pl.mid.bm == 0 || pingpong_us(m, n, k) < 0.9 * pl.mid.us)));
+  if (pl.pingpong) pl.mid.bm = 0;
+  // the streaming kernels take whole 16-byte chunks of a row, the tiled ones whole stages
+  const int64_t whole = pl.skinny || pl.mid.bm > 0 ? 16 : kStageK;
   pl.ks = k % whole == 0 ? k : pl.kp;
+  pl.partial_bytes = pl.mid.bm > 0 && pl.mid.splits > 1
+                         ? static_cast<size_t>(round_up(4 * pl.mid.splits * m * n, 256)) : 0;
   // In place only when every row's byte offset fits the kernels' 32-bit
   // offsets: the span of the last row ends below 2 GiB.
   pl.pack_a = !(a_sk == 1 && a_sm % 8 == 0 && aligned16(a) && k % whole == 0 &&
@@ -709,10 +816,6 @@ Fp8Plan plan_fp8(const void* a, int64_t a_sm, int64_t a_sk, const void* w, int64
                 (n - 1) * w_sn + k < kMaxOperandBytes);
   pl.a_bytes = pl.pack_a ? static_cast<size_t>(round_up(2 * m * pl.kp, 256)) : 0;
   pl.w_bytes = pl.pack_w ? static_cast<size_t>(round_up(n * pl.kp, 256)) : 0;
-  // >= 192 tiles of 256 x 192 (the INT8 kernel's large-grid rule): the
-  // ping-pong GEMM, fp8 W converted exactly to A's 2-byte type in registers
-  const int64_t tiles = ((m + 255) / 256) * ((n + 191) / 192);
-  pl.pingpong = !pl.skinny && tiles >= 192 && 2 * m * pl.kp < kMaxOperandBytes;
   return pl;
 }
 
@@ -749,9 +852,11 @@ extern "C" int qg_fp8w_gemm(const void* a, int a_dtype, int64_t a_sm, int64_t a_
   if (!float_dtype(out_dtype) || (bias && !float_dtype(bias_dtype))) return hipErrorInvalidValue;
   if (m == 0 || n == 0) return hipSuccess;
   if (!out || (k > 0 && (!a || !w))) return hipErrorInvalidValue;
-  const Fp8Plan pl = plan_fp8(a, a_sm, a_sk, w, w_sn, w_sk, m, n, k);
-  if (pl.total() > 0 && (!workspace || workspace_bytes < pl.total() || !aligned16(workspace)))
+  Fp8Plan pl = plan_fp8(a, a_sm, a_sk, w, w_sn, w_sk, m, n, k);
+  if (pl.packed() > 0 && (!workspace || workspace_bytes < pl.packed() || !aligned16(workspace)))
     return hipErrorInvalidValue;
+  if (pl.partial_bytes > 0 && (!workspace || workspace_bytes < pl.total() || !aligned16(workspace)))
+    pl.mid.splits = 1;
   // 32-bit byte offsets inside the kernel
   if (2 * m * pl.kp >= kMaxOperandBytes * 2 || n * pl.kp >= kMaxOperandBytes) return hipErrorInvalidValue;
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -787,7 +892,7 @@ extern "C" int qg_fp8w_gemm(const void* a, int a_dtype, int64_t a_sm, int64_t a_
   p.bias_dtype = bias_dtype;
   p.out = out;
   p.out_dtype = out_dtype;
-  if (pl.skinny) {
+  if (pl.skinny || pl.mid.bm > 0) {
     qg::SkinnyArgs t{};
     t.a = p.a;
     t.a_sm = p.a_sm;
@@ -801,7 +906,9 @@ extern "C" int qg_fp8w_gemm(const void* a, int a_dtype, int64_t a_sm, int64_t a_
     t.bias_dtype = bias_dtype;
     t.out = out;
     t.out_dtype = out_dtype;
-    return qg::launch_skinny_fp8(t, p.a_f16 != 0, p.fp8_e5 != 0, s);
+    if (pl.skinny) return qg::launch_skinny_fp8(t, p.a_f16 != 0, p.fp8_e5 != 0, s);
+    return qg::launch_mid_fp8(qg::MidArgs{t, pl.mid.splits, ws + pl.packed()}, pl.mid.bm, p.a_f16 != 0, p.fp8_e5 != 0,
+                              s);
   }
   if (pl.pingpong && k > 0) {
     // every fp8 value is exact in fp16 and bf16: the 2-byte ping-pong GEMM with
@@ -825,6 +932,24 @@ extern "C" int qg_fp8w_gemm(const void* a, int a_dtype, int64_t a_sm, int64_t a_
     return qg::launch_f8w_gemm(g, p.a_f16 != 0, p.fp8_e5 != 0, s);
   }
   return qg::launch_wd_fp8(p, s);  // k == 0: no stage, out = bias (or 0)
+}
+
+extern "C" int qg_row_kernel_choice(int format, int group_size, int flags, int64_t m, int64_t n, int64_t k) {
+  if (m < 1 || n < 1 || k < 1) return 0;
+  qg::MidPlan mid{0, 1, 0.0};
+  if (format == QG_CHOICE_W4A16) {
+    if (!valid_w4_shape(n, k, group_size, flags)) return 0;
+    const W4Plan pl = plan_w4(m, n, k, group_size, flags);
+    if (pl.mid.bm == 0) return pl.dequant_bytes > 0 ? QG_CHOICE_DEQUANT : 0;
+    mid = pl.mid;
+  } else if (format == QG_CHOICE_FP8) {
+    const Fp8Plan pl = plan_fp8(nullptr, round_up(k, 8), 1, nullptr, round_up(k, 16), 1, m, n, k);
+    if (pl.pingpong) return QG_CHOICE_PINGPONG;
+    mid = pl.mid;
+  } else if (format == QG_CHOICE_INT8) {
+    mid = plan_i8(nullptr, round_up(k, 16), 1, nullptr, 1, round_up(k, 16), m, n, k).mid;
+  }
+  return mid.bm > 0 ? (mid.splits << 16) | mid.bm : 0;
 }
 
 // ------------------------------------------------------------------- MoE

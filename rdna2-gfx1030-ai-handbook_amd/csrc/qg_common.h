@@ -174,6 +174,21 @@ __device__ __forceinline__ void dma16s(const void* sbase, uint32_t voff, uint32_
       : "memory");
 }
 
+// dma16s without the compiler barrier: LDS accesses may move across it, for
+// loops whose slot being filled is neither read nor written between the two
+// workgroup barriers around the copy.
+__device__ __forceinline__ void dma16s_free(const void* sbase, uint32_t voff, uint32_t lds_addr) {
+  uint32_t saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %2, %3\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(saved)
+      : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(sbase));
+}
+
 // dma16s with the non-temporal hint, for operands streamed once per launch
 // (the W4A16 decode's weights: 7.84-7.95 -> 7.43-7.71 us at cfg2 M = 1, one
 // box, alternating runs, same bits).

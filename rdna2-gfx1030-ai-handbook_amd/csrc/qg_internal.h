@@ -231,6 +231,51 @@ hipError_t launch_skinny_fp8(const SkinnyArgs& p, bool f16a, bool e5, hipStream_
 bool skinny_w4_applies(const W4Args& p);
 hipError_t launch_skinny_w4(const W4Args& p, hipStream_t stream);
 
+// Middling row counts (mid_gemm.hip): the operands as above, K split over
+// `splits` workgroups with partial tiles [splits][M][N] (4 bytes) when > 1.
+struct MidArgs {
+  SkinnyArgs op;
+  int splits;
+  void* partial;
+};
+
+constexpr int64_t kMidMaxRows = 2048;
+constexpr int64_t kMidMinK = 1024;  // shorter K has no stages to run ahead of
+enum MidKind { MID_FP8 = 0, MID_I8 = 1, MID_W4 = 2 };
+struct MidPlan {
+  int bm;      // tile rows; 0: the kernel does not apply
+  int splits;
+  double us;   // the model's time
+};
+MidPlan plan_mid(int kind, int group, int64_t m, int64_t n, int64_t k);
+// LDS bytes of an unsplit INT4 call.
+int64_t mid_w4_lds(int bm, int group, int64_t k);
+hipError_t launch_mid_fp8(const MidArgs& p, int bm, bool f16a, bool e5, hipStream_t stream);
+hipError_t launch_mid_i8(const MidArgs& p, hipStream_t stream);
+hipError_t launch_mid_w4(const W4Args& a, int bm, int splits, void* partial, hipStream_t stream);
+// INT4 operands (nk layout) of the streaming kernels.
+inline SkinnyArgs skinny_args(const W4Args& p) {
+  SkinnyArgs t{};
+  t.a = p.a;
+  t.a_sm = p.a_sm;
+  t.w = p.w;
+  t.w_sn = p.K / 2;
+  t.M = p.M;
+  t.N = p.N;
+  t.K = p.K;
+  t.flags = p.flags;
+  t.ng = p.ng;
+  t.zw = p.zw;
+  t.scales = p.scales;
+  t.scale_f32 = p.scale_f32;
+  t.zeros = p.zeros;
+  t.bias = p.bias;
+  t.bias_dtype = p.bias_dtype;
+  t.out = p.out;
+  t.out_dtype = p.out_dtype;
+  return t;
+}
+
 hipError_t launch_wd_w4(const WdArgs& p, hipStream_t stream);
 hipError_t launch_pack_rows_u16(const uint16_t* src, int64_t s_r, int64_t s_k, int64_t rows, int64_t K,
                                 uint16_t* dst, int64_t k_pad, hipStream_t stream);

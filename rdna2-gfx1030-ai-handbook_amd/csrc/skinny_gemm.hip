@@ -17,9 +17,7 @@
 //  * A lane reads 16 weight bytes of one column per k-step group and puts them
 //    into K order with two-input row exchanges (swap16 / swap32), so that the
 //    activations are used as they lie in memory.
-//  * LDS rows hold 16-byte chunks permuted by an XOR with the row, chosen so
-//    that the lanes of one ds_read_b128 phase (0-3, 12-15, 20-23, 24-27, and
-//    so on) hit different banks.
+//  * LDS rows hold 16-byte chunks permuted by an XOR with the row (lds_row_xor).
 //  * The 8 partial tiles are summed through LDS in wave order.
 // fp8, N 12288, K 3072 (37.7 MB of weights, one box, rotated weight copies):
 // 9.6 us at M 16 and 8.0 us at M <= 4 = 3.9 and 4.7 TB/s, against 40.9 us for
@@ -30,47 +28,11 @@
 #include "qg_common.h"
 #include "qg_epilogue.h"
 #include "qg_internal.h"
+#include "qg_wformat.h"
 
 namespace qg {
 
 namespace {
-
-enum SkinnyFormat { SK_I8 = 0, SK_E4M3 = 1, SK_E5M2 = 2, SK_W4 = 3, SK_UINT4 = 4 };
-
-// 8 nibbles (K order; high: nibble 7 first) -> 8 fp16 256 + 4 u or bf16 128 + u.
-template <bool F16A>
-struct NibbleExpand {
-  uint32_t sel[4], mask, magic;
-  __device__ __forceinline__ explicit NibbleExpand(bool high) {
-    static_for<0, 4>([&](auto ic) {
-      constexpr uint32_t i = decltype(ic)::value;
-      // halves of register i: elements 2 i and 2 i + 1, from the word (bytes
-      // 0-3) and the word shifted right by 4 (bytes 4-7), 0x0c = zero byte
-      sel[i] = high ? (0x0C000C00u | ((3u - i) << 16) | (7u - i)) : (0x0C000C00u | ((4u + i) << 16) | i);
-    });
-    mask = F16A ? 0x00F000F0u : 0x000F000Fu;
-    magic = F16A ? 0x5C005C00u : 0x43004300u;
-    asm volatile("" : "+v"(mask), "+v"(magic));
-  }
-  __device__ __forceinline__ i32x4 operator()(uint32_t w) const {
-    const uint32_t lo = F16A ? w << 4 : w, hi = F16A ? w : w >> 4;
-    i32x4 r;
-    static_for<0, 4>([&](auto i) {
-      r[int(i)] = static_cast<int>((__builtin_amdgcn_perm(hi, lo, sel[int(i)]) & mask) | magic);
-    });
-    return r;
-  }
-};
-
-template <bool F16A>
-__device__ __forceinline__ f32x4 mfma_half(const i32x4& a, const i32x4& b, const f32x4& c) {
-  if constexpr (F16A)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
-                                                  0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
-                                                   0, 0);
-}
 
 // RP: activation rows held in LDS (4, 8 or 16 >= M; fragment rows past RP
 // repeat row RP - 1). G: INT4 group size. D: ring depth.
@@ -126,8 +88,8 @@ __global__ __launch_bounds__(64 * C::NW) void k_skinny_gemm(SkinnyArgs p) {
   constexpr int APC = 1024 / C::AROW, ASL = C::AROW / 16;  // rows per copy, slots per row
   constexpr int WPC = 1024 / C::WROW, WSL = C::WROW / 16;
   uint32_t aoff[C::A_COPIES], woff[C::W_COPIES];
-  auto a_xor = [&](int row) __attribute__((always_inline)) { return C::I8 ? 2 * ((row >> 1) & 3) : (row & 15); };
-  auto w_xor = [&](int c) __attribute__((always_inline)) { return C::W4 ? (-(c >> 2)) & 3 : 2 * ((c >> 1) & 3); };
+  auto a_xor = [&](int row) __attribute__((always_inline)) { return lds_row_xor<C::AROW>(row); };
+  auto w_xor = [&](int c) __attribute__((always_inline)) { return lds_row_xor<C::WROW>(c); };
   const int a_slot = lane % ASL, w_slot = lane % WSL;
   static_for<0, C::A_COPIES>([&](auto i) {
     const int row = APC * i + lane / ASL;
@@ -218,13 +180,7 @@ __global__ __launch_bounds__(64 * C::NW) void k_skinny_gemm(SkinnyArgs p) {
         static_for<0, CT>([&](auto t) {
           w[t] = w_frag(t, 4 * u + q);
           if (tail && C::KS * c + 64 * u + 16 * q >= p.K) w[t] = zero4;
-          // 16 q .. 16 q + 15 -> 32 h + 8 q .. + 7 for step h
-          int w0 = w[t][0], w1 = w[t][1], w2 = w[t][2], w3 = w[t][3];
-          swap16(w0, w2);
-          swap32(w0, w2);
-          swap16(w1, w3);
-          swap32(w1, w3);
-          w[t] = i32x4{w0, w1, w2, w3};
+          w[t] = k_order_bytes(w[t]);
         });
         static_for<0, 2>([&](auto h) {
           constexpr int H = decltype(h)::value;
@@ -244,14 +200,7 @@ __global__ __launch_bounds__(64 * C::NW) void k_skinny_gemm(SkinnyArgs p) {
       const uint32_t* const zpar = reinterpret_cast<const uint32_t*>(par) + spart;
       i32x4 w[CT];
       static_for<0, CT>([&](auto t) {
-        w[t] = w_frag(t, q);
-        // words 4 q + j -> 4 j + q
-        int w0 = w[t][0], w1 = w[t][1], w2 = w[t][2], w3 = w[t][3];
-        swap16(w0, w1);
-        swap16(w2, w3);
-        swap32(w0, w2);
-        swap32(w1, w3);
-        w[t] = i32x4{w0, w1, w2, w3};
+        w[t] = k_order_words(w_frag(t, q));
       });
       f32x4 asum = {0, 0, 0, 0};
       static_for<0, 4>([&](auto j) {
@@ -262,8 +211,6 @@ __global__ __launch_bounds__(64 * C::NW) void k_skinny_gemm(SkinnyArgs p) {
         }
         const i32x4 a = a_frag(4 * J + q);
         asum = mfma_half<C::F16A>(a, ones, asum);
-        // steps 0 .. 3 of the exchanged words: w0, w1 hold words 0-3 and 4-7,
-        // w2, w3 words 8-11 and 12-15
         static_for<0, CT>([&](auto t) {
           acc[t] = mfma_half<C::F16A>(a, expand(static_cast<uint32_t>(w[t][J]) ^ wxor), acc[t]);
         });
@@ -469,24 +416,7 @@ bool skinny_w4_applies(const W4Args& p) {
 
 hipError_t launch_skinny_w4(const W4Args& p, hipStream_t stream) {
   if (!skinny_w4_applies(p)) return hipErrorInvalidValue;
-  SkinnyArgs t{};
-  t.a = p.a;
-  t.a_sm = p.a_sm;
-  t.w = p.w;
-  t.w_sn = p.K / 2;
-  t.M = p.M;
-  t.N = p.N;
-  t.K = p.K;
-  t.flags = p.flags;
-  t.ng = p.ng;
-  t.zw = p.zw;
-  t.scales = p.scales;
-  t.scale_f32 = p.scale_f32;
-  t.zeros = p.zeros;
-  t.bias = p.bias;
-  t.bias_dtype = p.bias_dtype;
-  t.out = p.out;
-  t.out_dtype = p.out_dtype;
+  const SkinnyArgs t = skinny_args(p);
   return p.a_f16 ? launch_skinny_w4_t<true>(t, p.group, stream) : launch_skinny_w4_t<false>(t, p.group, stream);
 }
 

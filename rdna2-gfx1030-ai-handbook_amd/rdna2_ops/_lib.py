@@ -38,6 +38,9 @@ W4_SIGNED_NIBBLES = 1
 W4_ORDER_HIGH = 2
 W4_LAYOUT_KN = 4
 W4_ZEROS_PACKED = 8
+# enum qg_choice_format, qg_choice
+CHOICE_W4A16, CHOICE_FP8, CHOICE_INT8 = range(3)
+CHOICE_DEQUANT, CHOICE_PINGPONG = 1, 2
 # enum qg_moe_epilogue, QG_MOE_TILE_ROWS
 MOE_EPI_I32 = 0
 MOE_EPI_SILU_MUL = 1
@@ -71,6 +74,7 @@ SIGNATURES = {
     "qg_w4a16_gemm_workspace_bytes": (_sz, [_i64, _i64, _i64, _i, _i]),
     "qg_w4a16_gemm": (_i, [_p, _i, _i64, _i64, _i64, _p, _i64, _i, _i, _p, _i, _p, _p, _i, _p, _i,
                            _p, _sz, _p]),
+    "qg_row_kernel_choice": (_i, [_i, _i, _i, _i64, _i64, _i64]),
     "qg_w4a8_gemm": (_i, [_p, _i64, _i64, _i64, _p, _i64, _i, _i, _p, _i, _p, _p, _i64, _p, _p, _i, _p, _i,
                           _p]),
     "qg_fp8_decode": (_i, [_p, _i, _i64, _i64, _i64, _i64, _p, _i, _p]),
@@ -154,6 +158,17 @@ def skinny_tiles(n: int, a_copies: int, w_copies: int, allowed=(1, 2, 3)) -> int
     """Column tiles of 16 per workgroup of the few-row kernel, as skinny_tiles
     in csrc/skinny_gemm.hip picks them."""
     return min(allowed, key=lambda ct: (-(-(-(-n // (16 * ct))) // 256) * (a_copies + ct * w_copies), ct))
+
+
+def mid_metadata(variant: str, choice: int, fmt: int, f16: bool, group: int = 128) -> dict:
+    """Metadata of the multi-stage kernel (csrc/mid_gemm.hip) behind a
+    qg_row_kernel_choice value past the two named ones."""
+    rows, splits = choice & 0xffff, choice >> 16
+    meta = kernel_metadata(variant, (rows, 128, 128), "k_mid_gemmINS0_6MidCfgILi{}ELb{}ELi{}E".format(
+        fmt, int(f16), rows) + ("" if fmt < 3 else "Li{}ELi{}E".format(
+            4 if rows == 32 or (rows == 64 and group == 128) else 3, group)))
+    meta["k_splits"] = splits
+    return meta
 
 
 @functools.lru_cache(maxsize=1)

@@ -177,20 +177,24 @@ def fp8_weight_gemm(a, w, *, bias=None, method="upcast", prepared=None, tile=(64
         raise ValueError("Unsupported tile or warp count")
     result = _fused(a, w, bias, w_scale)
     if metadata is not None:
-        # the C ABI's choice: up to 16 rows the streaming kernel; >= 192 tiles of 256 x 192 run the 2-byte
+        # the C ABI's choice: up to 16 rows the streaming kernel; up to 2048
+        # the multi-stage kernel where it is faster; else grids of tiles of
+        # 256 x 192 (from 192 of them always) run the 2-byte
         # ping-pong GEMM with fp8 W stages converted exactly to A's type in
         # registers; smaller grids the fused decode kernel (256 x 128 tiles
         # from four of them per CU)
         m, n = a.shape[0], w.shape[0]
         f16 = int(a.dtype == torch.float16)
-        kp = -(-a.shape[1] // 128) * 128
         if m <= 16:
             rows = 4 if m <= 4 else 8 if m <= 8 else 16
             ct = _lib.skinny_tiles(n, rows // 4, 2)
             variant, tile_used = "fp8w_skinny", (rows, 16 * ct, 128)
             hint = "k_skinny_gemmINS0_9SkinnyCfgILi{}ELb{}ELi{}ELi{}E".format(
                 2 if w.dtype == torch.float8_e5m2 else 1, f16, rows, ct)
-        elif (-(-m // 256)) * (-(-n // 192)) >= 192 and 2 * m * kp < 2 ** 31:
+        elif (choice := _lib.library().qg_row_kernel_choice(_lib.CHOICE_FP8, 0, 0, m, n, a.shape[1])) > 2:
+            meta = _lib.mid_metadata("fp8w_mid", choice, 2 if w.dtype == torch.float8_e5m2 else 1, f16)
+            variant, tile_used, hint = "fp8w_mid", meta["tile"], meta["symbol"]
+        elif choice == _lib.CHOICE_PINGPONG:
             variant = "fp8w_f16_pingpong" if f16 else "fp8w_bf16_pingpong"
             tile_used = (256, 192, 64)
             hint = "k_f8w_gemm_ppINS0_5F8GeoILi256ELi192ELi4ELi2ELi3EEELi{}ELb{}ELb{}E".format(

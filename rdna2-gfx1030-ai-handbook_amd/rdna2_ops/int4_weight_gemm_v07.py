@@ -347,12 +347,17 @@ def int4_linear_a16(a, p, *, bias=None, method="dequant", prepared=None, tile=(6
         bias = bias.contiguous()
     out = w4a16_gemm(a, p, bias)
     if return_kernel:
-        # the C ABI's choice: past 64 rows the dequant formulation from the
+        # the C ABI's choice: the multi-stage kernel, or past 64 rows the dequant formulation from the
         # group's tile threshold (K a multiple of 64), else the tiled MFMA kernel
         # (K a multiple of 128); up to 16 rows the one-row, decode and
         # streaming kernels; else skinny
         m = a.shape[0]
-        if _lib.library().qg_w4a16_gemm_workspace_bytes(m, p.n, p.k, p.group_size, p.flags) > 0:
+        choice = _lib.library().qg_row_kernel_choice(_lib.CHOICE_W4A16, p.group_size, p.flags, m, p.n, p.k)
+        uint4 = p.flags == _lib.W4_ZEROS_PACKED and p.group_size == 128 and p.scales.dtype == torch.bfloat16
+        if choice > _lib.CHOICE_PINGPONG:
+            return out, _lib.mid_metadata("w4a16_mid", choice, 4 if uint4 else 3, a.dtype == torch.float16,
+                                          p.group_size)
+        if choice == _lib.CHOICE_DEQUANT:
             # prefill grid at or past the group's threshold of 256 x 192 tiles
             # (192 at group 128, 64 at group 64, any at group 32): W
             # dequantised into the workspace, then the 2-byte ping-pong GEMM
@@ -373,7 +378,6 @@ def int4_linear_a16(a, p, *, bias=None, method="dequant", prepared=None, tile=(6
         if m <= 16 and not kn:
             if _gemv1_applies(a, p):
                 return out, _lib.kernel_metadata("w4a16_gemv1", (1, 32, 512), "k_w4_gemv1")
-            uint4 = p.flags == _lib.W4_ZEROS_PACKED and p.group_size == 128 and p.scales.dtype == torch.bfloat16
             ng = p.k // p.group_size
             if (uint4 and ng % 4 == 0 and -(-(-(-p.k // 128)) // 8) == 4 and m > 1
                     and p.n >= (8192 if m <= 4 else 12288)):

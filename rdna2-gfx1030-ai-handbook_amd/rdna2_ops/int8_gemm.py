@@ -134,20 +134,25 @@ def _launch(a, b, a_scale, b_scale, bias, *, tile, num_warps, num_stages, group_
     _lib.check(status, "qg_int8_gemm")
     if not return_kernel:
         return out
-    # the C ABI's choice: up to 16 rows the streaming kernel; >= 192 tiles of
+    # the C ABI's choice: up to 16 rows the streaming kernel; K split over
+    # workgroups where 128 x 128 tiles are few; >= 192 tiles of
     # 256 x 192 the persistent 8-wave ping-pong kernel, smaller grids the
     # 4-wave 128 x 128 one (K stage 128)
+    choice = lib.qg_row_kernel_choice(_lib.CHOICE_INT8, 0, 0, m, n, k)
+    partials = -(-4 * (choice >> 16) * m * n // 256) * 256
     if m <= 16 and k > 0:
         rows = 8 if m <= 8 else 16
         ct = _lib.skinny_tiles(n, rows // 8, 2)
         meta = _lib.kernel_metadata("int8_mfma_16x16x64_skinny", (rows, 16 * ct, 128),
                                     "k_skinny_gemmINS0_9SkinnyCfgILi0ELb0ELi{}ELi{}E".format(rows, ct))
+    elif choice > 0:
+        meta = _lib.mid_metadata("int8_mfma_16x16x64_split", choice, 0, False)
     elif (-(-m // 256)) * (-(-n // 192)) >= 192:
         meta = _lib.kernel_metadata("int8_mfma_32x32x32_pingpong", (256, 192, 128),
                                     "k_i8_gemm_ppINS0_5I8GeoILi256ELi192E")
     else:
         meta = _lib.kernel_metadata("int8_mfma_32x32x32", (128, 128, 128), "k_i8_gemmINS0_5I8GeoILi128ELi128E")
-    meta.update(packed_operands=ws_bytes > 0, requested_tile=list(tile), epilogue_flags=flags,
+    meta.update(packed_operands=ws_bytes > partials, requested_tile=list(tile), epilogue_flags=flags,
                 requested_wrapped=bool(wrapped), requested_partial_dot=bool(partial_dot))
     return out, meta
 

@@ -1,0 +1,164 @@
+"""The multi-stage kernel (17 to 2048 rows, K >= 1024) on the GPU: edges of its
+row tiles, splits of K and ragged K, each weight format against its oracle."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import case
+from oracle import fp8 as o8
+from oracle import int4 as o4
+from oracle import int8 as oi
+from test_fp8_gpu import check, codes_tensor
+from test_w4_gpu import act_values, check_product
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (17, 130, 1024), (32, 257, 1040), (33, 1, 4096), (64, 300, 12304), (65, 4096, 1152), (200, 1000, 2064),
+    (333, 129, 3072), (1000, 700, 1024), (1030, 140, 1536), (40, 50, 1025),
+])
+@pytest.mark.parametrize("e5,adtype", [(False, torch.bfloat16), (True, torch.float16)])
+def test_fp8_shapes(cuda, m, n, k, e5, adtype):
+    """Row tiles of 32 to 128, splits, a last stage of a few chunks, packed
+    operands (K % 16 != 0), strided rows, scale and bias."""
+    from rdna2_ops.fp8_weight_gemm_v06 import fp8_weight_gemm
+    case(f"mid fp8 {m}x{n}x{k} e5={e5} {adtype}")
+    rng = np.random.default_rng(m * 1000 + n + k)
+    codes = rng.integers(0, 256, (n, k)).astype(np.uint8)
+    dec = o8.decode_bits(codes, e5)
+    codes[~np.isfinite(dec) | (np.abs(dec) > 4)] = 0x30
+    a = torch.from_numpy(rng.standard_normal((m, k + 8)).astype(np.float32)).to(adtype)[:, :k]
+    scale = torch.from_numpy(rng.uniform(0.5, 2, n).astype(np.float32))
+    bias = torch.from_numpy(rng.standard_normal(n).astype(np.float32)).to(adtype)
+    md = {}
+    y = fp8_weight_gemm(a.to(cuda), codes_tensor(codes, e5, cuda), bias=bias.to(cuda), method="fused_dot2",
+                        w_scale=scale.to(cuda), metadata=md)
+    assert md["variant"] == "fp8w_mid" and md["vgpr"] is not None and md["vgpr_spills"] == 0, md
+    a64, w64 = a.double().numpy(), o8.decode_bits(codes, e5).astype(np.float64)
+    s64, b64 = scale.double().numpy(), bias.double().numpy()
+    check(y, (a64 @ w64.T) * s64 + b64, (np.abs(a64) @ np.abs(w64).T) * s64 + np.abs(b64), adtype, "mid fp8")
+
+
+@pytest.mark.parametrize("rows", [32, 64])
+def test_fp8_one_hot_rows(cuda, rows):
+    """One-hot activation rows read every K position of a stage and of a tail
+    back exactly, on both tile heights."""
+    from rdna2_ops.fp8_weight_gemm_v06 import fp8_weight_gemm
+    case(f"mid fp8 one-hot {rows}")
+    codes = np.arange(256, dtype=np.uint8)
+    codes = codes[np.isfinite(o8.decode_bits(codes, False))]
+    n, k = (4096 if rows == 64 else 64), 1104
+    w = codes[(np.arange(n)[:, None] * 7 + np.arange(k)[None, :]) % len(codes)].astype(np.uint8)
+    dec, wt = o8.decode_bits(w, False), codes_tensor(w, False, cuda)
+    for k0 in range(0, k, 368):
+        a = torch.zeros(368, k, dtype=torch.bfloat16)
+        a[torch.arange(368), k0 + torch.arange(368)] = 1
+        y = fp8_weight_gemm(a.to(cuda), wt, method="fused_dot2")
+        assert np.array_equal(y.float().cpu().numpy(), dec[:, k0:k0 + 368].T.astype(np.float32)), k0
+
+
+def test_fp8_values_past_k(cuda):
+    """Weight bytes after the last K element (NaN codes) do not reach the result."""
+    from rdna2_ops.fp8_weight_gemm_v06 import fp8_weight_gemm
+    case("mid fp8 NaN past K")
+    n, k, pitch = 24, 1040, 1280
+    store = np.full((n, pitch), 0x7f, np.uint8)
+    store[:, :k] = 0x38  # 1.0
+    w = codes_tensor(store, False, cuda)[:, :k]
+    y = fp8_weight_gemm(torch.ones(20, k, dtype=torch.bfloat16, device=cuda), w, method="fused_dot2")
+    assert torch.equal(y.float().cpu(), torch.full((20, n), float(k)))
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 130, 1088), (64, 300, 4096), (65, 4100, 1152), (333, 257, 2048),
+                                   (700, 1030, 1024), (1024, 1100, 3072)])
+@pytest.mark.parametrize("g", o4.GROUPS)
+@pytest.mark.parametrize("sym,order,adtype", [(True, "low", torch.float16), (False, "high", torch.bfloat16)])
+def test_int4_shapes(cuda, m, n, k, g, sym, order, adtype):
+    """Signed INT4 (nk): row tiles, splits, a last stage of fewer groups, both
+    nibble orders, bias. Where the dequant formulation stays the faster one the
+    product is held to the rounded weights' bound by the 1e-2 x RMS bar only."""
+    from rdna2_ops import int4_weight_gemm_v07 as w4
+    k = k // g * g
+    case(f"mid int4 {m}x{n}x{k} g{g} sym={sym} {order} {adtype}")
+    gen = torch.Generator().manual_seed(m + n + k + g)
+    w = torch.randn(n, k, generator=gen) * 0.02
+    a = torch.randn(m, k + 8, generator=gen).to(adtype)[:, :k]
+    b = (torch.randn(n, generator=gen) * 0.1).to(adtype)
+    p = w4.pack_int4(w.to(cuda), group_size=g, symmetric=sym, order=order)
+    cen = w4.unpack_int4(p, dtype=torch.int8).cpu().numpy().astype(np.int32)
+    av, s = act_values(a), p.scales.cpu().numpy()
+    y64 = o4.w4a16_linear(av, cen, s, g, act_values(b))
+    y, md = w4.int4_linear_a16(a.to(cuda), p, bias=b.to(cuda), method="dot2", return_kernel=True)
+    if md["variant"] == "w4a16_mid":
+        assert md["vgpr"] is not None and md["vgpr_spills"] == 0, md
+        check_product(y, y64, o4.w4a16_linear(np.abs(av), np.ones_like(cen), s, g), adtype, f"mid int4 {m}x{n}x{k} g{g}")
+    else:
+        err = np.abs(y.float().cpu().numpy() - y64)
+        assert (err <= 1e-2 * np.sqrt(np.mean(y64 ** 2)) + 2.0 ** -8 * np.abs(y64)).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(20, 140, 14336), (48, 4097, 1152), (96, 520, 4096), (512, 1000, 2048)])
+@pytest.mark.parametrize("adtype", [torch.float16, torch.bfloat16])
+def test_uint4_shapes(cuda, m, n, k, adtype):
+    from rdna2_ops import int4_weight_gemm_v07 as w4
+    case(f"mid uint4 {m}x{n}x{k} {adtype}")
+    gen = torch.Generator().manual_seed(m + n + k)
+    w = torch.randn(n, k, generator=gen) * 0.02
+    a = torch.randn(m, k, generator=gen).to(adtype)
+    p = w4.pack_uint4(w.to(cuda), group_size=128)
+    cen = w4.unpack_int4(p, dtype=torch.int8).cpu().numpy().astype(np.int32)
+    av, s = act_values(a), p.scales.float().cpu().numpy()
+    y, md = w4.int4_linear_a16(a.to(cuda), p, method="dot2", return_kernel=True)
+    assert md["variant"] == "w4a16_mid" and md["vgpr"] is not None
+    check_product(y, o4.w4a16_linear(av, cen, s, 128), o4.w4a16_linear(np.abs(av), np.ones_like(cen), s, 128),
+                  adtype, f"mid uint4 {m}x{n}x{k}")
+
+
+def test_int4_without_workspace(cuda):
+    """A call without the workspace of its partial tiles runs unsplit."""
+    from rdna2_ops import _lib
+    from rdna2_ops import int4_weight_gemm_v07 as w4
+    case("mid int4 no workspace")
+    gen = torch.Generator().manual_seed(5)
+    m, n, k = 100, 260, 4096
+    p = w4.pack_uint4((torch.randn(n, k, generator=gen) * 0.02).to(cuda), group_size=128)
+    a = torch.randn(m, k, generator=gen).to(torch.bfloat16).to(cuda)
+    lib, P = _lib.library(), _lib.ptr
+    assert lib.qg_w4a16_gemm_workspace_bytes(m, n, k, 128, p.flags) > 0
+    out = torch.empty(m, n, device=cuda)
+    _lib.check(lib.qg_w4a16_gemm(P(a), _lib.BF16, k, m, k, P(p.data), n, 128, p.flags, P(p.scales), _lib.BF16,
+                                 P(p.zeros), None, 0, P(out), _lib.F32, None, 0, _lib.stream_of(a)), "qg_w4a16_gemm")
+    ref = w4.w4a16_gemm(a, p, out_dtype=torch.float32)
+    assert (out - ref).abs().max().item() <= 1e-4 * ref.abs().max().item()  # fp32 sums in another order
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 140, 6160), (64, 300, 12288), (65, 1000, 4096), (130, 257, 6160),
+                                   (256, 3072, 8192), (300, 513, 8192)])
+def test_int8_split_shapes(cuda, m, n, k):
+    """int32 sums of split K bit-exact, and the epilogue orders of the second
+    launch; without workspace the tiled kernel gives the same bits."""
+    from rdna2_ops import _lib
+    from rdna2_ops.int8_gemm import int8_gemm_dequant, int8_matmul
+    case(f"mid int8 {m}x{n}x{k}")
+    g = torch.Generator().manual_seed(m * 31 + n * 7 + k)
+    a = torch.randint(-128, 128, (m, k), generator=g, dtype=torch.int8)
+    w = torch.randint(-128, 128, (n, k), generator=g, dtype=torch.int8)
+    sa, sb = torch.rand(m, generator=g) * 0.02 + 0.001, torch.rand(n, generator=g) * 0.02 + 0.001
+    bias = torch.randn(n, generator=g)
+    acc = oi.int8_matmul(a.numpy(), np.ascontiguousarray(w.numpy().T))
+    ag, wg, sag, sbg, bg = a.to(cuda), w.to(cuda), sa.to(cuda), sb.to(cuda), bias.to(cuda)
+    assert np.array_equal(int8_matmul(ag, wg.T).cpu().numpy(), acc)
+    y, md = int8_gemm_dequant(ag, wg.T, sag, sbg, bg, out_dtype=torch.float16, return_kernel=True)
+    assert md["variant"] == "int8_mfma_16x16x64_split" and md["k_splits"] > 1 and md["vgpr"] is not None, md
+    ref = oi.epilogue_f(acc, sa.numpy(), sb.numpy(), bias.numpy(), out="f16")
+    assert np.array_equal(y.float().cpu().numpy(), np.asarray(oi.round_to(ref, "f16"), np.float32))
+    y = int8_gemm_dequant(ag, wg.T, sag, sbg, bg, out_dtype=torch.bfloat16, epilogue_order="eager")
+    ref = oi.epilogue_e(acc, sa.numpy(), sb.numpy(), bias.numpy(), out="bf16")
+    assert np.array_equal(y.float().cpu().numpy(), np.asarray(oi.round_to(ref, "bf16"), np.float32))
+    if k % 128 == 0:
+        out = torch.empty(m, n, dtype=torch.int32, device=cuda)
+        P = _lib.ptr
+        _lib.check(_lib.library().qg_int8_gemm(P(ag), k, 1, P(wg), 1, k, m, n, k, None, None, 0, None, 0, P(out),
+                                               _lib.I32, 0, None, 0, _lib.stream_of(ag)), "qg_int8_gemm")
+        assert np.array_equal(out.cpu().numpy(), acc)
