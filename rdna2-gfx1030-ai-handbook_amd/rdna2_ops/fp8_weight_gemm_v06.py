@@ -32,6 +32,12 @@ _FP8 = (torch.float8_e4m3fn, torch.float8_e5m2)
 _ACT = (torch.float16, torch.bfloat16)
 
 
+def _span(t):
+    """Elements between the first and the last of a 2-D tensor."""
+    (m, k), (sm, sk) = t.shape, t.stride()
+    return (m - 1) * sm + (k - 1) * sk
+
+
 def _weight(w):
     """Contract of fp8_weight_gemm_v06.py:100-106 (arch: gfx950)."""
     if w.ndim != 2 or w.dtype not in _FP8:
@@ -39,7 +45,7 @@ def _weight(w):
     if w.device.type != "cuda":
         raise ValueError("This explicit implementation targets HIP gfx950")
     _lib.require_gfx950(w)
-    if min(w.shape) <= 0 or min(w.stride()) <= 0 or sum((n - 1) * s for n, s in zip(w.shape, w.stride())) >= 2 ** 31:
+    if min(w.shape) <= 0 or min(w.stride()) <= 0 or _span(w) >= 2 ** 31:
         raise ValueError("Nonempty positive strides and signed-32-bit address span required")
 
 
@@ -91,15 +97,16 @@ def _fused(a, w, bias, w_scale):
     m, k = a.shape
     n = w.shape[0]
     out = torch.empty((m, n), dtype=a.dtype, device=a.device)
-    lib = _lib.library()
-    ws_bytes = lib.qg_fp8w_gemm_workspace_bytes(_lib.ptr(a), a.stride(0), a.stride(1), _lib.ptr(w),
-                                                w.stride(0), w.stride(1), m, n, k)
-    wsp, wsn = _lib.ws_ptr(_lib.workspace(ws_bytes, a.device))
+    lib, code = _lib.library(), _lib.DTYPE_CODE
+    a_ptr, w_ptr, (a_sm, a_sk), (w_sn, w_sk) = a.data_ptr(), w.data_ptr(), a.stride(), w.stride()
+    ws_bytes = lib.qg_fp8w_gemm_workspace_bytes(a_ptr, a_sm, a_sk, w_ptr, w_sn, w_sk, m, n, k)
+    ws = _lib.workspace(ws_bytes, a.device)
+    wsp, wsn = _lib.ws_ptr(ws)
+    a_code = code[a.dtype]
     _lib.check(lib.qg_fp8w_gemm(
-        _lib.ptr(a), _lib.DTYPE_CODE[a.dtype], a.stride(0), a.stride(1), m, k, _lib.ptr(w),
-        _lib.DTYPE_CODE[w.dtype], w.stride(0), w.stride(1), n, _lib.ptr(w_scale), _lib.ptr(bias),
-        _lib.DTYPE_CODE[bias.dtype] if bias is not None else 0, _lib.ptr(out), _lib.DTYPE_CODE[a.dtype],
-        wsp, wsn, _lib.stream_of(a)), "qg_fp8w_gemm")
+        a_ptr, a_code, a_sm, a_sk, m, k, w_ptr, code[w.dtype], w_sn, w_sk, n, _lib.ptr(w_scale), _lib.ptr(bias),
+        code[bias.dtype] if bias is not None else 0, out.data_ptr(), a_code, wsp, wsn, _lib.stream_of(a)),
+        "qg_fp8w_gemm")
     return out
 
 
@@ -133,7 +140,7 @@ def fp8_weight_gemm(a, w, *, bias=None, method="upcast", prepared=None, tile=(64
             or getattr(torch.autograd.forward_ad, "_current_level", -1) >= 0
             or torch.is_grad_enabled() and (a.requires_grad or w.requires_grad)):
         raise ValueError("Only explicit eager inference is supported")
-    if min(a.shape) <= 0 or min(a.stride()) <= 0 or sum((n - 1) * s for n, s in zip(a.shape, a.stride())) >= 2 ** 31:
+    if min(a.shape) <= 0 or min(a.stride()) <= 0 or _span(a) >= 2 ** 31:
         raise ValueError("Nonempty positive-stride activation required")
     m, k = a.shape
     n = w.shape[0]

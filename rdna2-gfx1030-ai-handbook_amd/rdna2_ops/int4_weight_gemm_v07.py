@@ -190,9 +190,12 @@ def unpack_int4_cpu(p, *, floating=True):
 def _eager(*tensors):
     if (torch.compiler.is_compiling() or torch.cuda.is_current_stream_capturing()
             or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
-            or torch._C._are_functorch_transforms_active()
-            or torch.is_grad_enabled() and any(t.requires_grad for t in tensors)):
+            or torch._C._are_functorch_transforms_active()):
         raise ValueError("Explicit eager inference only")
+    if torch.is_grad_enabled():
+        for t in tensors:
+            if t.requires_grad:
+                raise ValueError("Explicit eager inference only")
 
 
 def _storage(n, k, group_size, layout, signed, zeros_packed, scale_dtype, device):
@@ -240,25 +243,36 @@ def pack_uint4(w, *, group_size=128):
     return _pack(w, group_size, False, "nk", "low", False, True, torch.bfloat16)
 
 
-def _validate(p):
-    """Contract of int4_weight_gemm_v07.py:433-447 (arch: gfx950)."""
+_SCALE_DTYPES = (torch.float32, torch.bfloat16)
+
+
+def _validate_storage(p):
+    """Contract of int4_weight_gemm_v07.py:433-447 (arch: gfx950), without the eager check."""
     if not isinstance(p, PackedInt4) or p.data.device.type != "cuda":
         raise ValueError("PackedInt4 on gfx950 required")
-    _lib.require_gfx950(p.data)
-    if (p.group_size not in _GROUPS or min(p.n, p.k) <= 0 or p.k % p.group_size or p.n * p.k >= 2 ** 31
+    data, n, k, group = p.data, p.n, p.k, p.group_size
+    _lib.require_gfx950(data)
+    if (group not in _GROUPS or min(n, k) <= 0 or k % group or n * k >= 2 ** 31
             or p.layout not in ("nk", "kn") or p.order not in ("low", "high")
-            or p.data.dtype != torch.int32 or not p.data.is_contiguous()
-            or tuple(p.data.shape) != ((p.n, p.k // 8) if p.layout == "nk" else (p.k // 8, p.n))):
+            or data.dtype != torch.int32 or not data.is_contiguous()
+            or data.shape != ((n, k // 8) if p.layout == "nk" else (k // 8, n))):
         raise ValueError("Invalid packed shape/storage")
-    ng = p.k // p.group_size
-    zshape = (p.n, (ng + 7) // 8) if p.zeros_packed else (p.n, ng)
-    scale_dtypes = (torch.float32, torch.bfloat16)
-    for t, dtypes, shape in ((p.scales, scale_dtypes, (p.n, ng)), (p.zeros, (torch.int32,), zshape),
-                             (p.sums, (torch.int32,), (p.n, ng))):
-        if t.device != p.data.device or t.dtype not in dtypes or tuple(t.shape) != shape or not t.is_contiguous():
-            raise ValueError("Invalid scale/zero/sum storage")
-    if p.data.data_ptr() % 16:
+    ng = k // group
+    scales, zeros, sums, device = p.scales, p.zeros, p.sums, data.device
+    if (scales.device != device or scales.dtype not in _SCALE_DTYPES or scales.shape != (n, ng)
+            or not scales.is_contiguous()
+            or zeros.device != device or zeros.dtype != torch.int32
+            or zeros.shape != ((n, (ng + 7) // 8) if p.zeros_packed else (n, ng)) or not zeros.is_contiguous()
+            or sums.device != device or sums.dtype != torch.int32 or sums.shape != (n, ng)
+            or not sums.is_contiguous()):
+        raise ValueError("Invalid scale/zero/sum storage")
+    if data.data_ptr() % 16:
         raise ValueError("Packed words must be 16-byte aligned")
+
+
+def _validate(p):
+    """Contract of int4_weight_gemm_v07.py:433-447 (arch: gfx950)."""
+    _validate_storage(p)
     _eager(p.data, p.scales)
 
 
@@ -310,13 +324,15 @@ def w4a16_gemm(a, p, bias=None, *, out_dtype=None):
     out = torch.empty((m, p.n), device=a.device, dtype=out_dtype)
     if m == 0:
         return out
-    lib = _lib.library()
-    ws_bytes = lib.qg_w4a16_gemm_workspace_bytes(m, p.n, k, p.group_size, p.flags)
-    wsp, wsn = _lib.ws_ptr(_lib.workspace(ws_bytes, a.device))
+    lib, flags, code = _lib.library(), p.flags, _lib.DTYPE_CODE
+    # up to 16 rows no kernel needs workspace
+    ws_bytes = lib.qg_w4a16_gemm_workspace_bytes(m, p.n, k, p.group_size, flags) if m > 16 else 0
+    ws = _lib.workspace(ws_bytes, a.device)
+    wsp, wsn = _lib.ws_ptr(ws)
     _lib.check(lib.qg_w4a16_gemm(
-        _lib.ptr(a), _lib.DTYPE_CODE[a.dtype], a.stride(0), m, k, _lib.ptr(p.data), p.n, p.group_size,
-        p.flags, _lib.ptr(p.scales), _lib.DTYPE_CODE[p.scales.dtype], _lib.ptr(p.zeros), _lib.ptr(bias),
-        _lib.DTYPE_CODE[bias.dtype] if bias is not None else 0, _lib.ptr(out), _lib.DTYPE_CODE[out_dtype],
+        a.data_ptr(), code[a.dtype], a.stride(0), m, k, p.data.data_ptr(), p.n, p.group_size,
+        flags, p.scales.data_ptr(), code[p.scales.dtype], p.zeros.data_ptr(), _lib.ptr(bias),
+        code[bias.dtype] if bias is not None else 0, out.data_ptr(), code[out_dtype],
         wsp, wsn, _lib.stream_of(a)), "qg_w4a16_gemm")
     return out
 
@@ -325,8 +341,8 @@ def int4_linear_a16(a, p, *, bias=None, method="dequant", prepared=None, tile=(6
                     num_warps=4, return_kernel=False):
     """fp16 (or bf16) activation and output: decode + library GEMM, prepared
     library GEMM, or the fused dot2 kernel (int4_weight_gemm_v07.py:540-564)."""
-    _validate(p)
-    _eager(a)
+    _validate_storage(p)
+    _eager(p.data, p.scales, a)
     if a.dtype not in (torch.float16, torch.bfloat16) or a.ndim != 2 or a.shape[1] != p.k or a.device != p.data.device:
         raise ValueError("Matching FP16 activation [M,K] required")
     if min(a.stride()) <= 0 or a.shape[0] * p.n >= 2 ** 31:

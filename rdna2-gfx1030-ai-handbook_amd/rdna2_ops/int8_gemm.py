@@ -40,6 +40,9 @@ _MAX_K = 131071
 _ROT_MAX_K = 16384  # QG_ROT_MAX_K: the ConvRot prologue holds one fp32 row in LDS
 
 
+_TILE = (32, 64, 64)  # the default tile of the operators below
+
+
 def _validate(a, b, tile, num_warps, num_stages, group_m):
     """Contract of rdna2-ops/rdna2_ops/int8_gemm.py:131-149 (arch: gfx950)."""
     if a.ndim != 2 or b.ndim != 2 or a.shape[1] != b.shape[0]:
@@ -49,11 +52,11 @@ def _validate(a, b, tile, num_warps, num_stages, group_m):
     if a.device.type != "cuda" or b.device != a.device:
         raise ValueError("Inputs must share a HIP device")
     _lib.require_gfx950(a)
-    if any(s < 0 for s in a.stride() + b.stride()):
+    if min(a.stride() + b.stride()) < 0:
         raise ValueError("Negative strides are unsupported")
     if a.shape[1] > _MAX_K:
         raise ValueError("K could overflow signed INT32 for arbitrary signed INT8 inputs")
-    if len(tile) != 3 or any(v < 16 or v > 256 or v & (v - 1) for v in tile):
+    if tile is not _TILE and (len(tile) != 3 or any(v < 16 or v > 256 or v & (v - 1) for v in tile)):
         raise ValueError("Tile dimensions must be powers of two in [16,256]")
     if num_warps not in (4, 8) or num_stages not in (1, 2, 3) or group_m not in (1, 2, 4, 8):
         raise ValueError("Unsupported launch configuration")
@@ -93,20 +96,21 @@ def _launch(a, b, a_scale, b_scale, bias, *, tile, num_warps, num_stages, group_
     if rounding not in ("separate", "fused"):
         raise ValueError("rounding must be separate or fused")
     if dequant:
+        device, grad = a.device, torch.is_grad_enabled()
         for value, size, label in ((a_scale, m, "a_scale"), (b_scale, n, "b_scale")):
             if not isinstance(value, torch.Tensor):
                 raise TypeError(label + " must be a device tensor")
-            if value.device != a.device or value.dtype != torch.float32 or not value.is_contiguous():
+            if value.device != device or value.dtype != torch.float32 or not value.is_contiguous():
                 raise ValueError(label + " must be contiguous FP32 on the input device")
             if value.numel() != size and not (label == "b_scale" and value.numel() == 1):
                 raise ValueError(label + " has the wrong number of elements")
-            if torch.is_grad_enabled() and value.requires_grad:
+            if grad and value.requires_grad:
                 raise ValueError("Autograd is unsupported")
         if bias is not None:
-            if (bias.device != a.device or bias.numel() != n or not bias.is_contiguous()
+            if (bias.device != device or bias.numel() != n or not bias.is_contiguous()
                     or bias.dtype not in (torch.float32, torch.float16, torch.bfloat16)):
                 raise ValueError("Bias must be a contiguous floating point vector of length N")
-            if torch.is_grad_enabled() and bias.requires_grad:
+            if grad and bias.requires_grad:
                 raise ValueError("Autograd is unsupported")
         if out_dtype not in _OUT_DTYPES:
             raise ValueError("out_dtype must be float32, float16 or bfloat16")
@@ -120,17 +124,19 @@ def _launch(a, b, a_scale, b_scale, bias, *, tile, num_warps, num_stages, group_
     if m == 0 or n == 0:
         return (out, None) if return_kernel else out
     lib = _lib.library()
-    ws_bytes = lib.qg_int8_gemm_workspace_bytes(
-        _lib.ptr(a), a.stride(0), a.stride(1), _lib.ptr(b), b.stride(0), b.stride(1), m, n, k)
+    a_sm, a_sk = a.stride()
+    b_sk, b_sn = b.stride()
+    a_ptr, b_ptr = a.data_ptr(), b.data_ptr()
+    ws_bytes = lib.qg_int8_gemm_workspace_bytes(a_ptr, a_sm, a_sk, b_ptr, b_sk, b_sn, m, n, k)
     ws = _lib.workspace(ws_bytes, a.device)
     wsp, wsn = _lib.ws_ptr(ws)
     status = lib.qg_int8_gemm(
-        _lib.ptr(a), a.stride(0), a.stride(1), _lib.ptr(b), b.stride(0), b.stride(1), m, n, k,
-        _lib.ptr(a_scale) if dequant else None, _lib.ptr(b_scale) if dequant else None,
+        a_ptr, a_sm, a_sk, b_ptr, b_sk, b_sn, m, n, k,
+        a_scale.data_ptr() if dequant else None, b_scale.data_ptr() if dequant else None,
         b_scale.numel() if dequant else 0,
         _lib.ptr(bias) if dequant else None,
         _lib.DTYPE_CODE[bias.dtype] if (dequant and bias is not None) else 0,
-        _lib.ptr(out), _lib.DTYPE_CODE[odt], flags, wsp, wsn, _lib.stream_of(a))
+        out.data_ptr(), _lib.DTYPE_CODE[odt], flags, wsp, wsn, _lib.stream_of(a))
     _lib.check(status, "qg_int8_gemm")
     if not return_kernel:
         return out
@@ -157,7 +163,7 @@ def _launch(a, b, a_scale, b_scale, bias, *, tile, num_warps, num_stages, group_
     return out, meta
 
 
-def int8_matmul(a, b, *, tile=(32, 64, 64), num_warps=4, num_stages=1,
+def int8_matmul(a, b, *, tile=_TILE, num_warps=4, num_stages=1,
                 group_m=4, return_kernel=False, wrapped=False, partial_dot=False):
     """Exact INT8 -> INT32 matmul; accepts both [K,N] layouts without copying.
 
@@ -170,7 +176,7 @@ def int8_matmul(a, b, *, tile=(32, 64, 64), num_warps=4, num_stages=1,
                    return_kernel=return_kernel, wrapped=wrapped, partial_dot=partial_dot)
 
 
-def int8_gemm_dequant(a, b, a_scale, b_scale, bias=None, *, tile=(32, 64, 64),
+def int8_gemm_dequant(a, b, a_scale, b_scale, bias=None, *, tile=_TILE,
                       num_warps=4, num_stages=1, group_m=4,
                       rounding="separate", return_kernel=False, wrapped=False, partial_dot=False,
                       out_dtype=torch.float32, activation=None, epilogue_order="reference"):
@@ -230,7 +236,7 @@ def w8a8_linear(x, weight, weight_scale, bias=None, *, out_dtype=None, activatio
     if k > _MAX_K:
         raise ValueError("K could overflow signed INT32 for arbitrary signed INT8 inputs")
     n = weight.shape[0]
-    ws_scale = weight_scale.reshape(-1)
+    ws_scale = weight_scale if weight_scale.ndim == 1 else weight_scale.reshape(-1)
     if (ws_scale.dtype != torch.float32 or ws_scale.device != x.device or not ws_scale.is_contiguous()
             or ws_scale.numel() not in (1, n)):
         raise ValueError("weight_scale must be contiguous FP32 with 1 or N elements")
@@ -258,7 +264,7 @@ def w8a8_linear(x, weight, weight_scale, bias=None, *, out_dtype=None, activatio
             raise ValueError("residual_scale must be contiguous FP32 with 1 or N elements")
     if weight.stride(1) != 1:
         weight = weight.contiguous()
-    x2 = x.reshape(-1, k)
+    x2 = x if x.ndim == 2 else x.reshape(-1, k)
     if k and x2.stride(1) != 1:
         x2 = x2.contiguous()
     m = x2.shape[0]
@@ -270,27 +276,27 @@ def w8a8_linear(x, weight, weight_scale, bias=None, *, out_dtype=None, activatio
     flags = _epilogue_flags("separate", activation, epilogue_order)
     out = torch.empty((m, n), device=x.device, dtype=out_dtype)
     if m and n:
-        lib = _lib.library()
-        need = lib.qg_w8a8_linear_workspace_bytes(_lib.ptr(weight), weight.stride(0), m, n, k)
-        ws = _lib.workspace(need, x.device)
+        lib, code = _lib.library(), _lib.DTYPE_CODE
+        w_ptr, w_sn = weight.data_ptr(), weight.stride(0)
+        ws = _lib.workspace(lib.qg_w8a8_linear_workspace_bytes(w_ptr, w_sn, m, n, k), x.device)
         wsp, wsn = _lib.ws_ptr(ws)
         rnd = _lib.ROUND_HALF_EVEN if rounding == "half_even" else _lib.ROUND_HALF_AWAY
-        bias_code = _lib.DTYPE_CODE[bias.dtype] if bias is not None else 0
+        bias_code = code[bias.dtype] if bias is not None else 0
         if convrot_groupsize is None and residual is None:
             status = lib.qg_w8a8_linear(
-                _lib.ptr(x2), _lib.DTYPE_CODE[x2.dtype], x2.stride(0), m, k, _lib.ptr(weight),
-                weight.stride(0), n, _lib.ptr(ws_scale), ws_scale.numel(), _lib.ptr(bias), bias_code,
-                _lib.ptr(out), _lib.DTYPE_CODE[out_dtype], rnd, flags, wsp, wsn, _lib.stream_of(x))
+                x2.data_ptr(), code[x2.dtype], x2.stride(0), m, k, w_ptr, w_sn, n, ws_scale.data_ptr(),
+                ws_scale.numel(), _lib.ptr(bias), bias_code, out.data_ptr(), code[out_dtype], rnd, flags, wsp, wsn,
+                _lib.stream_of(x))
             _lib.check(status, "qg_w8a8_linear")
         else:
             status = lib.qg_w8a8_linear_ex(
-                _lib.ptr(x2), _lib.DTYPE_CODE[x2.dtype], x2.stride(0), m, k, _lib.ptr(weight),
-                weight.stride(0), n, _lib.ptr(ws_scale), ws_scale.numel(), _lib.ptr(bias), bias_code,
-                int(convrot_groupsize or 0), _lib.ptr(r2), _lib.DTYPE_CODE[r2.dtype] if r2 is not None else 0,
-                r2.stride(0) if r2 is not None else 0, _lib.ptr(rs), rs.numel() if rs is not None else 0,
-                _lib.ptr(out), _lib.DTYPE_CODE[out_dtype], rnd, flags, wsp, wsn, _lib.stream_of(x))
+                x2.data_ptr(), code[x2.dtype], x2.stride(0), m, k, w_ptr, w_sn, n, ws_scale.data_ptr(),
+                ws_scale.numel(), _lib.ptr(bias), bias_code, int(convrot_groupsize or 0), _lib.ptr(r2),
+                code[r2.dtype] if r2 is not None else 0, r2.stride(0) if r2 is not None else 0, _lib.ptr(rs),
+                rs.numel() if rs is not None else 0, out.data_ptr(), code[out_dtype], rnd, flags, wsp, wsn,
+                _lib.stream_of(x))
             _lib.check(status, "qg_w8a8_linear_ex")
-    return out.reshape(*x.shape[:-1], n)
+    return out if x.ndim == 2 else out.reshape(*x.shape[:-1], n)
 
 
 def _research_knobs(tile, num_warps, num_stages, group_m, wrapped, partial_dot):
@@ -299,7 +305,7 @@ def _research_knobs(tile, num_warps, num_stages, group_m, wrapped, partial_dot):
 
 
 @contextmanager
-def moss_int8_gemm_candidate(*, tile=(32, 64, 64), num_warps=4,
+def moss_int8_gemm_candidate(*, tile=_TILE, num_warps=4,
                              num_stages=1, group_m=4, wrapped=False, partial_dot=False):
     """Scoped MOSS research export: Kitchen's eager backend exports a linear whose
     INT8 product and fp32 epilogue are one ``int8_gemm_dequant`` launch in the
@@ -368,7 +374,7 @@ def _patientx_weight_scale(weight_scale, weight, device, per_row):
 
 
 @contextmanager
-def qwen_int8_gemm_candidate(patch_module=None, *, tile=(32, 64, 64),
+def qwen_int8_gemm_candidate(patch_module=None, *, tile=_TILE,
                              num_warps=4, num_stages=1, group_m=4, wrapped=False, partial_dot=False):
     """Scoped replacement of the patientx bridge's two GEMM wrappers
     (``triton_int8_linear`` and ``triton_int8_linear_per_row``) by

@@ -148,46 +148,57 @@ def moe_int8_forward(x: torch.Tensor, router_logits: torch.Tensor, weights: MoeI
     rows, tiles_n = rows_c.value, tiles_c.value
     logits = router_logits.float().contiguous()
     x = x.contiguous()
-    i32 = dict(dtype=torch.int32, device=dev)
-    experts = torch.empty(t, top_k, **i32)
-    rweights = torch.empty(t, top_k, dtype=torch.float32, device=dev)
-    counts = torch.empty(_lib.MOE_COUNTS_PER_EXPERT * e, **i32)
-    row_token = torch.empty(rows, **i32)
-    row_weight = torch.empty(rows, dtype=torch.float32, device=dev)
-    row_slot = torch.empty(rows, **i32)
-    tiles = torch.empty(tiles_n, 4, **i32)
     stream = _lib.stream_of(x)
     P = _lib.ptr
-    xq = torch.empty(t, h, dtype=torch.int8, device=dev)
-    xs = torch.empty(t, dtype=torch.float32, device=dev)
+    # The stages' tensors are parts of one allocation of this call, 256-byte
+    # aligned; only ``return_intermediates`` looks at them as tensors.
+    sizes = (("experts", 4 * t * top_k), ("weights", 4 * t * top_k), ("counts", 4 * _lib.MOE_COUNTS_PER_EXPERT * e),
+             ("row_token", 4 * rows), ("row_weight", 4 * rows), ("row_slot", 4 * rows), ("tiles", 16 * tiles_n),
+             ("xq", t * h), ("xs", 4 * t), ("h", 2 * rows * f), ("hq", rows * f), ("hs", 4 * rows),
+             ("y", 2 * t * top_k * h))
+    offset, total = {}, 0
+    for name, size in sizes:
+        offset[name] = total
+        total += (size + 255) & ~255
+    ws = _lib.workspace(total, dev)
+    base, _ = _lib.ws_ptr(ws)
+    at = {name: base + o for name, o in offset.items()}
     if h % 8 == 0 and h <= MOE_ROUTE_QUANT_MAX_H and x.data_ptr() % 16 == 0:
         # the routing launch quantizes x as well (bit-identical to qg_quant_rows_i8)
-        _lib.check(lib.qg_moe_dispatch_qx(P(logits), e, t, e, top_k, pad, P(experts), P(rweights), P(counts),
-                                          P(row_token), P(row_weight), P(row_slot), rows, P(tiles), tiles_n,
-                                          P(x), h, h, P(xq), h, P(xs), stream), "qg_moe_dispatch_qx")
+        _lib.check(lib.qg_moe_dispatch_qx(P(logits), e, t, e, top_k, pad, at["experts"], at["weights"], at["counts"],
+                                          at["row_token"], at["row_weight"], at["row_slot"], rows, at["tiles"], tiles_n,
+                                          P(x), h, h, at["xq"], h, at["xs"], stream), "qg_moe_dispatch_qx")
     else:
-        _lib.check(lib.qg_moe_dispatch(P(logits), e, t, e, top_k, pad, P(experts), P(rweights), P(counts),
-                                       P(row_token), P(row_weight), P(row_slot), rows, P(tiles), tiles_n, stream),
-                   "qg_moe_dispatch")
-        _quant_rows(x, xq, xs)
-    hbuf = torch.empty(rows, f, dtype=torch.bfloat16, device=dev)
-    _lib.check(lib.qg_moe_grouped_gemm(P(xq), h, t, P(row_token), rows, h, P(weights.w13), h, 2 * f * h, 2 * f, e,
-                                       P(tiles), tiles_n, P(xs), P(weights.s13), None, None, _lib.MOE_EPI_SILU_MUL,
-                                       P(hbuf), f, rows, stream), "qg_moe_grouped_gemm gate/up")
-    hq = torch.empty(rows, f, dtype=torch.int8, device=dev)
-    hs = torch.empty(rows, dtype=torch.float32, device=dev)
-    _quant_rows(hbuf, hq, hs)
-    y = torch.empty(t * top_k, h, dtype=torch.bfloat16, device=dev)
-    _lib.check(lib.qg_moe_grouped_gemm(P(hq), f, rows, None, rows, f, P(weights.w2), f, h * f, h, e, P(tiles),
-                                       tiles_n, P(hs), P(weights.s2), P(row_weight), P(row_slot),
-                                       _lib.MOE_EPI_ROUTE, P(y), h, t * top_k, stream), "qg_moe_grouped_gemm down")
+        _lib.check(lib.qg_moe_dispatch(P(logits), e, t, e, top_k, pad, at["experts"], at["weights"], at["counts"],
+                                       at["row_token"], at["row_weight"], at["row_slot"], rows, at["tiles"], tiles_n,
+                                       stream), "qg_moe_dispatch")
+        _lib.check(lib.qg_quant_rows_i8(P(x), _lib.BF16, h, 1, t, h, at["xq"], h, at["xs"], _lib.ROUND_HALF_EVEN,
+                                        stream), "qg_quant_rows_i8")
+    _lib.check(lib.qg_moe_grouped_gemm(at["xq"], h, t, at["row_token"], rows, h, P(weights.w13), h, 2 * f * h, 2 * f, e,
+                                       at["tiles"], tiles_n, at["xs"], P(weights.s13), None, None,
+                                       _lib.MOE_EPI_SILU_MUL, at["h"], f, rows, stream), "qg_moe_grouped_gemm gate/up")
+    _lib.check(lib.qg_quant_rows_i8(at["h"], _lib.BF16, f, 1, rows, f, at["hq"], f, at["hs"], _lib.ROUND_HALF_EVEN,
+                                    stream), "qg_quant_rows_i8")
+    _lib.check(lib.qg_moe_grouped_gemm(at["hq"], f, rows, None, rows, f, P(weights.w2), f, h * f, h, e, at["tiles"],
+                                       tiles_n, at["hs"], P(weights.s2), at["row_weight"], at["row_slot"],
+                                       _lib.MOE_EPI_ROUTE, at["y"], h, t * top_k, stream), "qg_moe_grouped_gemm down")
     out = torch.empty(t, h, dtype=torch.bfloat16, device=dev)
-    _lib.check(lib.qg_moe_combine(P(y), t, top_k, h, P(out), h, stream), "qg_moe_combine")
+    _lib.check(lib.qg_moe_combine(at["y"], t, top_k, h, P(out), h, stream), "qg_moe_combine")
     if not return_intermediates:
         return out
-    return out, {"experts": experts, "weights": rweights, "counts": counts, "row_token": row_token,
-                 "row_weight": row_weight, "row_slot": row_slot, "tiles": tiles, "xq": xq, "xs": xs, "h": hbuf,
-                 "hq": hq, "hs": hs, "y": y, "rows_max": rows}
+
+    def part(name, dtype, *shape):
+        start = at[name] - ws.data_ptr()
+        count = shape[0] * (shape[1] if len(shape) > 1 else 1)
+        return ws[start:start + count * dtype.itemsize].view(dtype).reshape(shape)
+
+    i32, f32, i8, b16 = torch.int32, torch.float32, torch.int8, torch.bfloat16
+    return out, {"experts": part("experts", i32, t, top_k), "weights": part("weights", f32, t, top_k),
+                 "counts": part("counts", i32, _lib.MOE_COUNTS_PER_EXPERT * e), "row_token": part("row_token", i32, rows),
+                 "row_weight": part("row_weight", f32, rows), "row_slot": part("row_slot", i32, rows),
+                 "tiles": part("tiles", i32, tiles_n, 4), "xq": part("xq", i8, t, h), "xs": part("xs", f32, t),
+                 "h": part("h", b16, rows, f), "hq": part("hq", i8, rows, f), "hs": part("hs", f32, rows),
+                 "y": part("y", b16, t * top_k, h), "rows_max": rows}
 
 
 def grouped_gemm_i32(a: torch.Tensor, row_token, tiles: torch.Tensor, w: torch.Tensor, rows_max: int) -> torch.Tensor:
