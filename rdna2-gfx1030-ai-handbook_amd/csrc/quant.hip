@@ -235,13 +235,40 @@ __global__ __launch_bounds__(256) void k_rot_quant_rows(const char* x, int64_t x
   if (t == 0) step_out[row] = step;
 }
 
-// Register-resident form of k_rot_quant_rows for K a multiple of 512 (up to
+// The value of lane l ^ D: DPP permutations inside rows of 16 lanes (quad
+// permutations for 1 and 2, a reversed quad then a reversed half row for 4, a
+// half-row rotation for 8), row exchanges for 16 and 32. ds_bpermute instead
+// (80 a lane at K 8192, group 256) bound the kernel by LDS: 1061 x 8192 fp32
+// 14.6 us, this form 13.1 us (the quantizer alone 9.3 us).
+template <int D>
+__device__ __forceinline__ float lane_xor(float x) {
+  const int i = __float_as_int(x);
+  int r;
+  if constexpr (D == 1) {
+    r = __builtin_amdgcn_mov_dpp(i, 0xB1, 0xf, 0xf, true);
+  } else if constexpr (D == 2) {
+    r = __builtin_amdgcn_mov_dpp(i, 0x4E, 0xf, 0xf, true);
+  } else if constexpr (D == 4) {
+    r = __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(i, 0x1B, 0xf, 0xf, true), 0x141, 0xf, 0xf, true);
+  } else if constexpr (D == 8) {
+    r = __builtin_amdgcn_mov_dpp(i, 0x128, 0xf, 0xf, true);
+  } else {
+    static_assert(D == 16 || D == 32, "lane distance");
+    int a = i, b = i;  // a: the lower rows of each pair in both, b: the upper ones
+    if constexpr (D == 16) swap16(a, b);
+    else swap32(a, b);
+    r = (threadIdx.x & D) != 0 ? a : b;
+  }
+  return __int_as_float(r);
+}
+
+// Register-resident form of k_rot_quant_rows for K a multiple of 8 (up to
 // QG_ROT_MAX_K) and groups of 8 to 512: one row per workgroup of NW = min(8,
-// K / 512) waves; lane t of the workgroup holds, in each of NS slots, the 8
+// ceil(K / 512)) waves; lane t of the workgroup holds, in each of NS slots, the 8
 // consecutive values 8 (s 64 NW + t) .. + 7 of the row as fp32. A group of G
 // values is G / 8 consecutive lanes of one slot (aligned), so the butterfly
 // stages h = 1, 2, 4 pair registers of a lane, and the stages h = 8 .. G / 2
-// pair register e of lanes h / 8 apart (__shfl_xor): the lower element of a
+// pair register e of lanes h / 8 apart (lane_xor): the lower element of a
 // pair becomes a + c and the upper a - c, with a the lower and c the upper
 // value — the operations, operands and stage order of the LDS form, so the
 // results are the same bits. Lanes past K hold zeros (whole groups, K % G ==
@@ -303,19 +330,23 @@ __global__ __launch_bounds__(512) void k_rot_quant_rows_reg(const char* x, int64
       }
     });
   });
-  // butterflies across lanes: h = 8 d for lane distance d = 1 .. G / 16
-  for (int d = 1; 8 * d < G; d <<= 1) {
-    const bool upper = (lane & d) != 0;
-    static_for<0, NS>([&](auto s_c) {
-      constexpr int S = decltype(s_c)::value;
-      static_for<0, 8>([&](auto e_c) {
-        constexpr int e = decltype(e_c)::value;
-        const float self = v[S][e];
-        const float other = __shfl_xor(self, d, 64);
-        v[S][e] = upper ? other - self : self + other;
+  // butterflies across lanes: h = 8 d for lane distance d = 1 .. G / 16. With s
+  // = -1 in the upper lane of a pair and 1 in the lower, other + s self is a - c
+  // and a + c (s self is exact, so the fma rounds once, like the sum)
+  static_for<0, 6>([&](auto ld_c) {
+    constexpr int D = 1 << decltype(ld_c)::value;
+    if (8 * D < G) {
+      const float sign = (lane & D) != 0 ? -1.0f : 1.0f;
+      static_for<0, NS>([&](auto s_c) {
+        constexpr int S = decltype(s_c)::value;
+        static_for<0, 8>([&](auto e_c) {
+          constexpr int e = decltype(e_c)::value;
+          const float self = v[S][e];
+          v[S][e] = __builtin_fmaf(sign, self, lane_xor<D>(self));
+        });
       });
-    });
-  }
+    }
+  });
   float amax = 0.0f;
   static_for<0, NS>([&](auto s_c) {
     constexpr int S = decltype(s_c)::value;
@@ -341,16 +372,17 @@ __global__ __launch_bounds__(512) void k_rot_quant_rows_reg(const char* x, int64
   if (t == 0) step_out[row] = step;
 }
 
-// The register form's contract (K % 512 == 0, groups 8 .. 512, 16-byte
+// The register form's contract (K % 8 == 0, groups 8 .. 512, 16-byte
 // aligned rows); its slot count per lane (at most 4: the launcher's largest
 // instantiation).
 static_assert(QG_ROT_MAX_K <= 4 * 512 * 8, "register ConvRot form: at most 4 slots of 8 values per lane");
+inline int64_t rot_waves(int64_t K) { return (K + 511) / 512 < 8 ? (K + 511) / 512 : 8; }
 inline int rot_reg_slots(const void* x, int x_dtype, int64_t x_sm, int64_t K, int G, int8_t* q, int64_t q_sm) {
   const int es = x_dtype == QG_F32 ? 4 : 2;
-  if (K % 512 != 0 || K > QG_ROT_MAX_K || G < 8 || G > 512) return 0;
+  if (K % 8 != 0 || K > QG_ROT_MAX_K || G < 8 || G > 512) return 0;
   if ((reinterpret_cast<uintptr_t>(x) & 15) != 0 || (x_sm * es) % 16 != 0) return 0;
   if ((reinterpret_cast<uintptr_t>(q) & 7) != 0 || q_sm % 8 != 0) return 0;
-  const int64_t nw = K / 512 < 8 ? K / 512 : 8;
+  const int64_t nw = rot_waves(K);
   return static_cast<int>((K + 512 * nw - 1) / (512 * nw));
 }
 
@@ -363,7 +395,7 @@ hipError_t launch_rot_quant_mode(const void* x, int x_dtype, int64_t x_sm, int64
   const int k = static_cast<int>(K), kp = static_cast<int>(k_pad);
   const int ns = rot_reg_slots(x, x_dtype, x_sm, K, G, q, q_sm);
   if (ns > 0) {
-    const dim3 block(static_cast<unsigned>(64 * (K / 512 < 8 ? K / 512 : 8)));
+    const dim3 block(static_cast<unsigned>(64 * rot_waves(K)));
 #define QG_ROT_REG(XT, NS)                                                                                      \
   hipLaunchKernelGGL((k_rot_quant_rows_reg<XT, MODE, NS>), grid, block, 0, stream, xp, x_sm, k, G, inv_sqrt_g, q, \
                      q_sm, kp, step)
