@@ -74,7 +74,7 @@ I8Plan plan_i8(const void* a, int64_t a_sm, int64_t a_sk, const void* b, int64_t
   pl.b_bytes = pl.pack_b ? static_cast<size_t>(round_up(n * pl.kp, 256)) : 0;
   pl.mid = qg::plan_mid(qg::MID_I8, 128, m, n, k);
   // a second launch costs the host about 4 us: it has to win clearly more
-  if (pl.mid.bm == 0 || pl.mid.splits == 1 || pl.mid.us + 10.0 > tiled_i8_us(m, n, k)) pl.mid = qg::MidPlan{0, 1, 0.0};
+  if (pl.mid.bm == 0 || pl.mid.splits == 1 || pl.mid.us + 6.0 > tiled_i8_us(m, n, k)) pl.mid = qg::MidPlan{0, 1, 0.0};
   pl.partial_bytes = pl.mid.bm > 0 ? static_cast<size_t>(round_up(4 * pl.mid.splits * m * n, 256)) : 0;
   return pl;
 }
