@@ -106,6 +106,14 @@ hipError_t launch_moe_dispatch(const MoeDispatchArgs& p, hipStream_t stream);
 hipError_t launch_moe_combine(const uint16_t* y, int T, int top_k, int H, uint16_t* out, int64_t out_sm,
                               hipStream_t stream);
 
+// Rows of row_bytes bytes, s_r bytes apart at any alignment, to rows of
+// dst_bytes (zeros past row_bytes), where packs_as_bytes holds: whole aligned
+// 16-byte pieces, few enough for a 32-bit index.
+inline bool packs_as_bytes(const void* dst, int64_t rows, int64_t dst_bytes) {
+  return dst_bytes % 16 == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0 && rows * (dst_bytes / 16) < (1ll << 31);
+}
+hipError_t launch_pack_rows_bytes(const void* src, int64_t s_r, int64_t rows, int64_t row_bytes, void* dst,
+                                  int64_t dst_bytes, hipStream_t stream);
 // dst[r, k] = src[r * s_r + k * s_k] for k < K, 0 for K <= k < k_pad.
 hipError_t launch_pack_rows_i8(const int8_t* src, int64_t s_r, int64_t s_k,
                                int64_t rows, int64_t K, int8_t* dst,

@@ -456,6 +456,8 @@ unsigned grid_for(int64_t total) {
 hipError_t launch_pack_rows_u16(const uint16_t* src, int64_t s_r, int64_t s_k, int64_t rows, int64_t K,
                                 uint16_t* dst, int64_t k_pad, hipStream_t stream) {
   if (rows * k_pad == 0) return hipSuccess;
+  if (s_k == 1 && packs_as_bytes(dst, rows, 2 * k_pad))
+    return launch_pack_rows_bytes(src, 2 * s_r, rows, 2 * K, dst, 2 * k_pad, stream);
   hipLaunchKernelGGL(k_pack_rows_u16, dim3(grid_for(rows * k_pad)), dim3(256), 0, stream, src, s_r, s_k, rows,
                      K, dst, k_pad);
   return hipGetLastError();
