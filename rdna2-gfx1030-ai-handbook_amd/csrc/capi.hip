@@ -1099,6 +1099,7 @@ extern "C" int qg_moe_grouped_gemm(const int8_t* a, int64_t a_sm, int64_t a_rows
   p.out_rows = static_cast<int>(out_rows);
   p.n_experts = n_experts;
   p.moe_epi = epilogue;
+  if (qg::moe_rows_applies(p)) return qg::launch_moe_rows(p, static_cast<hipStream_t>(stream));
   return qg::launch_i8_moe_gemm(p, static_cast<hipStream_t>(stream));
 }
 

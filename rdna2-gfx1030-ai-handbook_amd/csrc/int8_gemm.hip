@@ -1157,12 +1157,6 @@ __global__ __launch_bounds__(G::THREADS, 1) void k_f8w_gemm_pp(I8GemmArgs p) {
 constexpr int kBufferWord3 = 0x00020000;
 constexpr uint32_t kOobOffset = 0x7FFFFFF0u;
 
-__device__ __forceinline__ float silu(float g) {
-#pragma clang fp contract(off)
-  // g / (1 + e^-g) with the hardware exp2 and reciprocal (a few ulps)
-  return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f));
-}
-
 // Candidate work items per workgroup of the grouped kernel: their table
 // entries are copied into LDS at the start (launch_i8_moe_gemm rejects plans
 // that would need more).

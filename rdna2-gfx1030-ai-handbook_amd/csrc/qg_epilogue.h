@@ -26,6 +26,12 @@ __device__ __forceinline__ float gelu_tanh(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
+__device__ __forceinline__ float silu(float g) {
+#pragma clang fp contract(off)
+  // g / (1 + e^-g) with the hardware exp2 and reciprocal (a few ulps)
+  return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f));
+}
+
 // Raw storage bits of bias[col] (fp32, fp16 or bf16) and their fp32 value.
 __device__ __forceinline__ uint32_t load_bias_bits(const void* bias, int dtype, int col) {
   if (dtype == QG_F32) return static_cast<const uint32_t*>(bias)[col];

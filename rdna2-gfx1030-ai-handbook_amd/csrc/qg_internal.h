@@ -60,6 +60,10 @@ hipError_t launch_i8_gemm_stages(const I8GemmArgs& p, hipStream_t stream);
 
 hipError_t launch_i8_gemm(const I8GemmArgs& p, hipStream_t stream);
 hipError_t launch_i8_moe_gemm(const I8GemmArgs& p, hipStream_t stream);
+// The same call with few routed rows per expert (moe_rows.hip).
+constexpr int kMoeFewRows = 16;
+bool moe_rows_applies(const I8GemmArgs& p);
+hipError_t launch_moe_rows(const I8GemmArgs& p, hipStream_t stream);
 // 2-byte (fp16 / bf16) A and W on the ping-pong main loop; p.a_sm / p.w_sn /
 // p.K in elements, a_scale null (1), b_scale per column or null (1).
 hipError_t launch_h16_gemm(const I8GemmArgs& p, bool f16a, hipStream_t stream);

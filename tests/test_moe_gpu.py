@@ -373,3 +373,81 @@ def test_moe_combine_slot_counts_and_row_widths(cuda, t, top_k, h, out_sm):
     exp_bits = torch.from_numpy(np.ascontiguousarray(exp)).bfloat16().view(torch.int16)
     assert torch.equal(got[:, :h], exp_bits)
     assert (got[:, h:] == -1).all()
+
+
+# few rows per expert (csrc/moe_rows.hip): one row; 8, 9 and 16 rows in every
+# expert (row tiles of 8 and 16, the last slot count of the route epilogue's
+# rule), 17 and 64 (repeated passes), 65 (past the rule)
+@pytest.mark.parametrize("t,e,h,f,top_k", [(1, 64, 256, 128, 8), (8, 8, 256, 128, 8), (9, 8, 640, 384, 8),
+                                           (16, 8, 2048, 128, 8), (17, 8, 256, 768, 8), (64, 8, 256, 128, 8),
+                                           (65, 8, 256, 128, 8)])
+def test_moe_few_rows(cuda, t, e, h, f, top_k):
+    case(f"moe few rows t{t} e{e} h{h} f{f} k{top_k}")
+    x, logits, wg, wu, wd = make_case(100 + t, t, e, h, f, top_k)
+    run_and_check(cuda, x, logits, wg, wu, wd, top_k, label=f"few rows t{t}")
+
+
+def test_moe_few_rows_skewed(cuda):
+    """64 rows of one expert, few per expert on average: four passes of both products."""
+    case("moe few rows skewed")
+    x, logits, wg, wu, wd = make_case(77, 64, 64, 256, 128, 2)
+    logits[:, 3] += 20.0
+    run_and_check(cuda, x, logits, wg, wu, wd, 2, label="few rows skewed")
+
+
+@pytest.mark.parametrize("n", [32, 96, 77])
+def test_moe_few_rows_table_and_edges(cuda, n):
+    """Entries that name no expert, one past the last, or rows outside the
+    operands are skipped, as is one past the count in use; column remainders
+    (N 77: int32 and route); padded output rows; route targets out of range."""
+    from rdna2_ops import _lib
+    case(f"moe few rows table n{n}")
+    rng = np.random.default_rng(n)
+    E, K, M = 4, 384, 48
+    a = rng.integers(-127, 128, (M, K), dtype=np.int8)
+    w = rng.integers(-127, 128, (E, n, K), dtype=np.int8)
+    sa = (rng.random(M, dtype=np.float32) * 0.02 + 0.001).astype(np.float32)
+    sb = (rng.random((E, n), dtype=np.float32) * 0.02 + 0.001).astype(np.float32)
+    rw = rng.random(M, dtype=np.float32).astype(np.float32)
+    slot = rng.permutation(M).astype(np.int32)
+    slot[[3, 20]] = -1
+    slot[[10, 30]] = M
+    tiles = np.array([[0, 0, 5, 6], [-1, 5, 9, 0], [2, 8, 25, 0], [4, 25, 30, 0], [1, 30, 38, 0],
+                      [3, 40, 49, 0], [3, 40, 48, 0]], np.int32)
+    valid = [(0, 0, 5), (2, 8, 25), (1, 30, 38)]
+    d = {k_: torch.from_numpy(v).to(cuda) for k_, v in
+         dict(a=a, w=w, sa=sa, sb=sb, rw=rw, slot=slot, tiles=tiles).items()}
+    out = torch.full((M, n + 1), -7, dtype=torch.int32, device=cuda)
+    _grouped_call(cuda, d["a"], d["w"], d["tiles"], None, None, None, None, _lib.MOE_EPI_I32, out)
+    exp = np.full((M, n + 1), -7, np.int64)
+    for e, r0, r1 in valid:
+        exp[r0:r1, :n] = a[r0:r1].astype(np.int64) @ w[e].T.astype(np.int64)
+    assert np.array_equal(out.cpu().numpy().astype(np.int64), exp)
+
+    exp_y = np.full((M, n + 3), np.nan, np.float32)
+    for e, r0, r1 in valid:
+        yv = om.down(a[r0:r1], sa[r0:r1], w[e], sb[e], rw[r0:r1])
+        for i, r in enumerate(range(r0, r1)):
+            if 0 <= slot[r] < M:
+                exp_y[slot[r], :n] = yv[i]
+    buf = torch.full((M, n + 3), -1, dtype=torch.int16, device=cuda)  # 0xFFFF: a bf16 NaN
+    y = buf.view(torch.bfloat16)
+    _grouped_call(cuda, d["a"], d["w"], d["tiles"], d["sa"], d["sb"], d["rw"], d["slot"], _lib.MOE_EPI_ROUTE, y)
+    assert np.array_equal(y.float().cpu().numpy(), exp_y, equal_nan=True)
+    if n % 32:
+        return
+    F = n // 2
+    g_rows = np.array([32 * (f // 16) + f % 16 for f in range(F)])
+    buf = torch.full((M, F + 1), -1, dtype=torch.int16, device=cuda)
+    h = buf.view(torch.bfloat16)
+    _grouped_call(cuda, d["a"], d["w"], d["tiles"], d["sa"], d["sb"], None, None, _lib.MOE_EPI_SILU_MUL, h)
+    exp_h = np.full((M, F + 1), np.nan, np.float32)
+    for e, r0, r1 in valid:
+        exp_h[r0:r1, :F] = om.gate_up(a[r0:r1], sa[r0:r1], w[e][g_rows], sb[e][g_rows], w[e][g_rows + 16],
+                                      sb[e][g_rows + 16])
+    vals = h.float().cpu().numpy()
+    assert np.array_equal(np.isnan(vals), np.isnan(exp_h))
+    hit = ~np.isnan(exp_h)
+    err = np.abs(vals[hit] - exp_h[hit])
+    # one bf16 ulp, as run_and_check's h
+    assert (err <= 2.0 ** -7 * np.abs(exp_h[hit]) + 1e-6).all(), err.max()
