@@ -451,3 +451,38 @@ def test_moe_few_rows_table_and_edges(cuda, n):
     err = np.abs(vals[hit] - exp_h[hit])
     # one bf16 ulp, as run_and_check's h
     assert (err <= 2.0 ** -7 * np.abs(exp_h[hit]) + 1e-6).all(), err.max()
+
+
+# one workgroup routes and dispatches up to 16 tokens; 17 take both launches, as
+# does a padding whose rows pass 8192; expert 0 takes a slot of every token
+@pytest.mark.parametrize("t,e,k,pad", [(1, 1, 1, 1), (1, 64, 64, 64), (2, 64, 8, 64), (15, 33, 5, 7), (16, 64, 8, 64),
+                                       (16, 8, 8, 1), (16, 2, 1, 4096), (16, 8, 2, 1024), (16, 4, 2, 4096),
+                                       (17, 64, 8, 64)])
+def test_moe_dispatch_few_tokens(cuda, t, e, k, pad):
+    from rdna2_ops import _lib
+    case(f"moe dispatch few t{t} e{e} k{k} pad{pad}")
+    logits = torch.randn(t, e, generator=torch.Generator().manual_seed(t * e + k))
+    if t > 2:
+        logits[:, 0] += 20.0
+    m = mod()
+    x, _, wg, wu, wd = make_case(3, t, e, 128, 128, k)
+    prep = m.prepare_moe_weights(wg.to(cuda), wu.to(cuda), wd.to(cuda))
+    _, it = m.moe_int8_forward(x.to(cuda), logits.to(cuda), prep, top_k=k, pad=pad, return_intermediates=True)
+    ex_o, w_o = om.route_topk(logits.numpy(), k)
+    assert np.array_equal(it["experts"].cpu().numpy(), ex_o)
+    # as run_and_check, plus exp2's argument x, which is rounded twice (difference
+    # and product): a relative error of 2 * 2^-24 * ln 2 * |x|
+    spread = float((logits.amax(1) - logits.amin(1)).max()) * 1.4427
+    np.testing.assert_allclose(it["weights"].cpu().numpy(), w_o, rtol=1e-6 + 2.0 ** -23 * 0.6932 * spread, atol=0)
+    counts, offsets, rows, rt_o, rs_o = om.dispatch(ex_o, e, pad=pad)
+    assert np.array_equal(it["counts"][:e].cpu().numpy(), counts)
+    assert np.array_equal(it["counts"][e:2 * e].cpu().numpy(), offsets)
+    rt, rs, rw = (it[name].cpu().numpy() for name in ("row_token", "row_slot", "row_weight"))
+    assert np.array_equal(rt[:rows], rt_o) and np.array_equal(rs[:rows], rs_o)
+    assert (rt[rows:] == -1).all() and (rs[rows:] == -1).all() and (rw[rs < 0] == 0).all()
+    assert np.array_equal(rw[rs >= 0], it["weights"].cpu().numpy().reshape(-1)[rs[rs >= 0]])
+    want = [(ei, int(o) + j, int(o) + int(c)) for ei, (c, o) in enumerate(zip(counts, offsets))
+            for j in range(0, (int(c) + pad - 1) // pad * pad, _lib.MOE_TILE_ROWS)]
+    tl = it["tiles"].cpu().numpy()
+    assert tl[0, 3] == len(want) and np.array_equal(tl[:len(want), :3], np.array(want))
+    assert (tl[len(want):, 0] == -1).all() and (tl[1:, 3] == 0).all()
