@@ -28,6 +28,7 @@
 #include "qg_common.h"
 #include "qg_epilogue.h"
 #include "qg_internal.h"
+#include "qg_w4_params.h"
 #include "qg_wformat.h"
 
 namespace qg {
@@ -57,14 +58,9 @@ struct SkinnyCfg {
   static_assert(LDS <= 160 * 1024, "LDS per CU");
 };
 
-// LDS words per column of the INT4 scales and zero points: odd, so that a
-// group's 16 columns lie in different banks. bf16 scales of a column may start
-// in the upper half of a word.
-__host__ __device__ __forceinline__ int skinny_scale_pitch(int ng, bool f32) { return (f32 ? ng : ng / 2 + 1) | 1; }
-__host__ __device__ __forceinline__ int skinny_zero_pitch(int ng, int zw, bool packed) { return (packed ? zw : ng) | 1; }
 inline int skinny_par_bytes(const SkinnyArgs& p, int cols) {
-  const int s = cols * skinny_scale_pitch(p.ng, p.scale_f32);
-  const int z = cols * skinny_zero_pitch(p.ng, p.zw, p.flags & QG_W4_ZEROS_PACKED);
+  const int s = cols * w4_scale_pitch(p.ng, p.scale_f32);
+  const int z = cols * w4_zero_pitch(p.ng, p.zw, p.flags & QG_W4_ZEROS_PACKED);
   return 4 * (((s + 63) & ~63) + ((z + 63) & ~63));
 }
 
@@ -122,24 +118,31 @@ __global__ __launch_bounds__(64 * C::NW) void k_skinny_gemm(SkinnyArgs p) {
   // 19 us).
   const bool zpacked = C::UINT4 || (p.flags & QG_W4_ZEROS_PACKED);
   const bool sf32 = !C::UINT4 && p.scale_f32;
-  const int sper = skinny_scale_pitch(p.ng, sf32), zper = skinny_zero_pitch(p.ng, p.zw, zpacked);
+  const int sper = w4_scale_pitch(p.ng, sf32), zper = w4_zero_pitch(p.ng, p.zw, zpacked);
   const int spart = (16 * CT * sper + 63) & ~63;  // words of the scale part
   if constexpr (C::W4) {
     const uint32_t par_addr = lds_addr_of(smem + C::PAR_AT);
-    // word e: word e % pitch of column e / pitch (padding re-reads a word that exists)
-    auto copy_words = [&](const void* base, int pitch, int used, uint32_t at, auto first)
-        __attribute__((always_inline)) {
+    // word e: word e % pitch of column e / pitch
+    auto copy_words = [&](int pitch, auto copy) __attribute__((always_inline)) {
       for (int w0 = 64 * wave; w0 < 16 * CT * pitch; w0 += 64 * C::NW) {
-        const int e = w0 + lane, cc = e / pitch, k = min(e - cc * pitch, used - 1);
-        dma4s(base, 4u * (first(static_cast<uint32_t>(min(n0 + cc, p.N - 1))) + k), at + 4 * w0);
+        const int e = w0 + lane, cc = e / pitch;
+        copy(static_cast<uint32_t>(min(n0 + cc, p.N - 1)), static_cast<uint32_t>(e - cc * pitch), 4u * w0);
       }
     };
-    // the words of a column's bf16 scales start at the one holding group 0
-    const uint32_t ng = p.ng;
-    const int sused = sf32 ? p.ng : (p.ng + 1) / 2;
-    copy_words(p.scales, sper, sused, par_addr, [&](uint32_t n) { return sf32 ? n * ng : (n * ng) >> 1; });
-    copy_words(p.zeros, zper, zpacked ? p.zw : p.ng, par_addr + 4 * spart,
-               [&](uint32_t n) { return n * static_cast<uint32_t>(zpacked ? p.zw : p.ng); });
+    if (!sf32 && (p.N * p.ng & 1)) {  // the last scale is half a word
+      copy_words(sper, [&](uint32_t n, uint32_t w, uint32_t to) __attribute__((always_inline)) {
+        const W4Read r = w4_scale_read(n, p.N, p.ng, false, w);
+        if (r.bytes == 2) dma2s(p.scales, r.offset, par_addr + to);
+        else dma4s(p.scales, r.offset, par_addr + to);
+      });
+    } else {
+      copy_words(sper, [&](uint32_t n, uint32_t w, uint32_t to) __attribute__((always_inline)) {
+        dma4s(p.scales, w4_scale_read(n, p.N, p.ng, sf32, w).offset, par_addr + to);
+      });
+    }
+    copy_words(zper, [&](uint32_t n, uint32_t w, uint32_t to) __attribute__((always_inline)) {
+      dma4s(p.zeros, w4_zero_read(n, zpacked ? p.zw : p.ng, w).offset, par_addr + 4 * spart + to);
+    });
   }
 
   acc_t acc[CT];
