@@ -282,6 +282,62 @@ __global__ __launch_bounds__(64 * C::NW, 1) void k_mid_gemm(MidArgs p) {
     }
   }
 
+  // ---- INT4: elements that are not finite ------------------------------------
+  // The loop sums a (MAGIC + UNIT u) and takes the zero point's share off each
+  // group's sum, which turns an infinite activation, or a sum past fp32's range,
+  // into NaN in every column. Such elements are summed again with the weights
+  // u - z themselves, the products that the dequantized weights give (finite
+  // elements keep their bits; the loop above is as it was without this).
+  if constexpr (C::W4) {
+    float off = 0.0f;  // NaN if some element of the lane is not finite
+    static_for<0, FM>([&](auto f) {
+      static_for<0, FN>([&](auto t) {
+        static_for<0, 4>([&](auto e) { off = __builtin_fmaf(total[f][t][int(e)], 0.0f, off); });
+      });
+    });
+    if (__builtin_expect(__any(off != 0.0f), 0)) static_for<0, FM>([&](auto f) {
+      static_for<0, FN>([&](auto t) {
+        bool lost[4];
+        static_for<0, 4>([&](auto e) { lost[int(e)] = !(fabsf(total[f][t][int(e)]) < __builtin_inff()); });
+        if (!__any(lost[0] || lost[1] || lost[2] || lost[3])) return;
+        constexpr int STEPS = C::G / 32;  // of a group
+        const int cc = wc * 16 * FN + 16 * t + col;
+        const char* const ar = static_cast<const char*>(o.a) +
+                               2 * static_cast<int64_t>(min(m0 + (wr * FM + f) * 16 + col, o.M - 1)) * o.a_sm;
+        const uint32_t* const wr32 = reinterpret_cast<const uint32_t*>(static_cast<const char*>(o.w) +
+                                                                       min(n0 + cc, o.N - 1) * o.w_sn);
+        const float2* const par = reinterpret_cast<const float2*>(smem + C::PAR_AT) + cc;
+        const int groups = min(S * C::SPC, o.ng - g0);
+        f32x4 again = {0, 0, 0, 0};
+        for (int g = 0; g < groups; ++g) {
+          const float2 sz = par[g * C::BN];
+          f32x4 sum = {0, 0, 0, 0};
+          static_for<0, STEPS>([&](auto j) {
+            const int step = (g0 + g) * STEPS + j;
+            const i32x4 a = *reinterpret_cast<const i32x4*>(ar + 64 * step + 16 * q);
+            i32x4 b = expand(wr32[4 * step + q] ^ wxor);
+            static_for<0, 4>([&](auto i) {
+              const uint32_t x = static_cast<uint32_t>(b[int(i)]);
+              const uint16_t lo = static_cast<uint16_t>(x), hi = static_cast<uint16_t>(x >> 16);
+              uint32_t l, h;  // u - z (times UNIT), exact
+              if constexpr (C::F16A) {
+                l = f32_to_f16(f16_to_f32(lo) - sz.y);
+                h = f32_to_f16(f16_to_f32(hi) - sz.y);
+              } else {
+                l = f32_to_bf16(bf16_to_f32(lo) - sz.y);
+                h = f32_to_bf16(bf16_to_f32(hi) - sz.y);
+              }
+              b[int(i)] = static_cast<int>(l | h << 16);
+            });
+            sum = mfma_half<C::F16A>(a, b, sum);
+          });
+          static_for<0, 4>([&](auto e) { again[int(e)] = __builtin_fmaf(sz.x, sum[int(e)], again[int(e)]); });
+        }
+        static_for<0, 4>([&](auto e) { total[f][t][int(e)] = lost[int(e)] ? again[int(e)] : total[f][t][int(e)]; });
+      });
+    });
+  }
+
   // ---- output: row 4 q + e of block f, column col of block t -----------------
   static_for<0, FN>([&](auto t) {
     const int nn = n0 + wc * 16 * FN + 16 * t + col;

@@ -115,6 +115,44 @@ def test_uint4_shapes(cuda, m, n, k, adtype):
                   adtype, f"mid uint4 {m}x{n}x{k}")
 
 
+@pytest.mark.parametrize("m,n,k,g", [
+    (300, 513, 4096, 32), (100, 140, 1120, 32), (300, 4096, 4096, 64), (100, 300, 1088, 64), (1024, 1030, 2048, 128),
+    (100, 260, 4096, 128),
+])
+@pytest.mark.parametrize("sym,adtype", [(True, torch.float16), (False, torch.bfloat16)])
+def test_int4_infinite_activations(cuda, m, n, k, g, sym, adtype):
+    """An infinite activation gives what the dequantized weights give: +-inf,
+    or NaN where the weight is zero or infinities of both signs meet; sums past
+    fp32's range on the way (bf16) stay finite, and the other rows' bits do not
+    change."""
+    from rdna2_ops import int4_weight_gemm_v07 as w4
+    case(f"mid int4 inf {m}x{n}x{k} g{g} sym={sym} {adtype}")
+    gen = torch.Generator().manual_seed(m + n + k + g)
+    p = w4.pack_int4((torch.randn(n, k, generator=gen) * 0.02).to(cuda), group_size=g, symmetric=sym)
+    w = (w4.unpack_int4(p, dtype=torch.int8).double().reshape(n, k // g, g) * p.scales.double()[..., None]).reshape(n, k)
+    a = torch.randn(m, k, generator=gen).to(adtype)
+    before = w4.w4a16_gemm(a.to(cuda), p)
+    rows = {1: {k - 3: float("inf")}, m // 2: {5: -float("inf")}, m - 1: {0: float("inf"), k // 2: float("inf")},
+            m - 2: {9: float("inf"), k - 1: -float("inf")}, 7: {11: float("nan")}}
+    for r, at in rows.items():
+        for c, v in at.items():
+            a[r, c] = v
+    if adtype == torch.bfloat16:
+        rows[3] = None
+        a[3] = torch.randn(k, generator=gen).bfloat16() * 2.0 ** 120
+    y, md = w4.int4_linear_a16(a.to(cuda), p, method="dot2", return_kernel=True)
+    assert md["variant"] == "w4a16_mid", md
+    rest = [r for r in range(m) if r not in rows]
+    assert torch.equal(y[rest], before[rest])
+    for r in rows:
+        ref = (a[r].double().to(cuda) * w).sum(-1)
+        got = y[r].double()
+        assert torch.equal(got.isnan(), ref.isnan()), r
+        assert torch.equal(got[got.isinf()], ref[ref.isinf()]) and torch.equal(got.isinf(), ref.isinf()), r
+    if adtype == torch.bfloat16:
+        assert ((got - ref).abs() <= 1e-2 * ref.square().mean().sqrt() + 2.0 ** -8 * ref.abs()).all()
+
+
 def test_int4_without_workspace(cuda):
     """A call without the workspace of its partial tiles runs unsplit."""
     from rdna2_ops import _lib
