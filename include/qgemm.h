@@ -269,12 +269,13 @@ int qg_w4_unpack(const int32_t* data, int64_t n, int64_t k, int group_size,
  * dequant formulation instead: W is dequantised once into the
  * workspace, (q - z) * s in fp32 rounded to the activation dtype, then a
  * 2-byte MFMA GEMM with fp32 accumulation runs on it; the workspace is then
- * 2 * n * k bytes (16-byte aligned), reported by
- * qg_w4a16_gemm_workspace_bytes, and required. nk weights with K >= 1024 and
- * up to 2048 rows keep the exact group sums instead where that is faster; K
- * may then be split over workgroups, with fp32 partial tiles in the workspace
- * that qg_w4a16_gemm_workspace_bytes reports (without it the call runs
- * unsplit). 0 on the other shapes.
+ * 2 * n * k bytes (16-byte aligned). nk weights with K >= 1024 and up to 2048
+ * rows keep the exact group sums instead where that is faster; K may then be
+ * split over workgroups, with fp32 partial tiles in the workspace.
+ * qg_w4a16_gemm_workspace_bytes reports what the fastest of these needs (0 on
+ * the other shapes). With less, the call takes the fastest that fits: unsplit,
+ * where the group parameters of K fit in LDS, or the dequant formulation. So
+ * 2 * n * k bytes always suffice; a call that has neither choice is refused.
  * a: [m, k] QG_F16 or QG_BF16, unit K stride, row stride a_sm (a multiple of 8
  * elements, 16-byte aligned base); w: 16-byte aligned; out: [m, n] contiguous
  * QG_F16 / QG_BF16 / QG_F32; bias NULL or [n] of bias_dtype; m * n < 2^31. */

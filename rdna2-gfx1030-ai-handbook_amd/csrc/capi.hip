@@ -75,7 +75,7 @@ I8Plan plan_i8(const void* a, int64_t a_sm, int64_t a_sk, const void* b, int64_t
   pl.mid = qg::plan_mid(qg::MID_I8, 128, m, n, k);
   // a second launch costs the host about 4 us: it has to win clearly more
   if (pl.mid.bm == 0 || pl.mid.splits == 1 || pl.mid.us + 6.0 > tiled_i8_us(m, n, k)) pl.mid = qg::MidPlan{0, 1, 0.0};
-  pl.partial_bytes = pl.mid.bm > 0 ? static_cast<size_t>(round_up(4 * pl.mid.splits * m * n, 256)) : 0;
+  pl.partial_bytes = pl.mid.bm > 0 ? qg::mid_partial_bytes(pl.mid.splits, m, n) : 0;
   return pl;
 }
 
@@ -600,17 +600,20 @@ struct W4Plan {
   qg::MidPlan mid;       // bm > 0: mid_gemm
   size_t dequant_bytes;  // > 0: dequant + ping-pong
   size_t total(int64_t m, int64_t n) const {
-    if (mid.bm > 0) return mid.splits > 1 ? static_cast<size_t>(round_up(4 * mid.splits * m * n, 256)) : 0;
-    return dequant_bytes;
+    return mid.bm > 0 ? qg::mid_partial_bytes(mid.splits, m, n) : dequant_bytes;
   }
 };
-W4Plan plan_w4(int64_t m, int64_t n, int64_t k, int group_size, int flags) {
+// room: workspace bytes at hand. A formulation that needs more is left out; the
+// dequant formulation is returned all the same (total() > room) where nothing
+// else takes the call.
+W4Plan plan_w4(int64_t m, int64_t n, int64_t k, int group_size, int flags, size_t room = SIZE_MAX) {
   W4Plan pl{qg::MidPlan{0, 1, 0.0}, w4_prefill_bytes(m, n, k, group_size)};
   if ((flags & QG_W4_LAYOUT_KN) || m <= qg::kSkinnyMaxRows || k < qg::kMidMinK) return pl;
-  pl.mid = qg::plan_mid(qg::MID_W4, group_size, m, n, k);
+  pl.mid = qg::plan_mid(qg::MID_W4, group_size, m, n, k, room);
   double before_us = 1.0e9;
   if (m <= kW4TiledMinRows) before_us = skinny_w4_us(m, n, k, group_size);
-  else if (pl.dequant_bytes > 0) before_us = 2.5 + n * k * 2.5 / 4.4e6 + pingpong_us(m, n, k);
+  else if (pl.dequant_bytes > 0 && pl.dequant_bytes <= room)
+    before_us = 2.5 + n * k * 2.5 / 4.4e6 + pingpong_us(m, n, k);
   if (pl.mid.us > 0.9 * before_us) pl.mid.bm = 0;
   return pl;
 }
@@ -704,17 +707,10 @@ extern "C" int qg_w4a16_gemm(const void* a, int a_dtype, int64_t a_sm, int64_t m
   p.bias_dtype = bias_dtype;
   p.out = out;
   p.out_dtype = out_dtype;
-  W4Plan pl = plan_w4(m, n, k, group_size, flags);
-  const size_t need = pl.total(m, n);
+  const size_t room = workspace && aligned16(workspace) ? workspace_bytes : 0;
+  const W4Plan pl = plan_w4(m, n, k, group_size, flags, room);
+  if (pl.total(m, n) > room) return hipErrorInvalidValue;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (need > 0 && (!workspace || workspace_bytes < need || !aligned16(workspace))) {
-    // the dequant formulation needs its workspace; without room for the
-    // partial tiles K is not split (up to 64 rows k_w4_skinny is faster then)
-    if (pl.mid.bm == 0) return hipErrorInvalidValue;
-    pl.mid.splits = 1;
-    if (m <= kW4TiledMinRows || qg::mid_w4_lds(pl.mid.bm, group_size, k) > 160 * 1024) pl.mid.bm = 0;
-    if (pl.mid.bm == 0 && pl.dequant_bytes > 0) return hipErrorInvalidValue;
-  }
   if (pl.mid.bm > 0) return qg::launch_mid_w4(p, pl.mid.bm, pl.mid.splits, workspace, s);
   // dequantise W into the workspace, then the 2-byte ping-pong GEMM (out = acc
   // + bias, one rounding)
@@ -806,8 +802,7 @@ Fp8Plan plan_fp8(const void* a, int64_t a_sm, int64_t a_sk, const void* w, int64
   // the streaming kernels take whole 16-byte chunks of a row, the tiled ones whole stages
   const int64_t whole = pl.skinny || pl.mid.bm > 0 ? 16 : kStageK;
   pl.ks = k % whole == 0 ? k : pl.kp;
-  pl.partial_bytes = pl.mid.bm > 0 && pl.mid.splits > 1
-                         ? static_cast<size_t>(round_up(4 * pl.mid.splits * m * n, 256)) : 0;
+  pl.partial_bytes = pl.mid.bm > 0 ? qg::mid_partial_bytes(pl.mid.splits, m, n) : 0;
   // In place only when every row's byte offset fits the kernels' 32-bit
   // offsets: the span of the last row ends below 2 GiB.
   pl.pack_a = !(a_sk == 1 && a_sm % 8 == 0 && aligned16(a) && k % whole == 0 &&

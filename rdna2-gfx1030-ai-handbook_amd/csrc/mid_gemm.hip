@@ -473,8 +473,9 @@ hipError_t launch_mid_w4_t(const MidArgs& p, int group, int bm, hipStream_t stre
 // box, which it meets within about 10 %: 3.5 us plus the stages of one
 // workgroup times the rounds of 256 workgroups times the time of a stage
 // (128 K elements; 15 % more where rounds overlap); a split adds 2.5 us and
-// its partial tiles at 4 TB/s. A split has to win by 10 %.
-MidPlan plan_mid(int kind, int group, int64_t m, int64_t n, int64_t k) {
+// its partial tiles at 4 TB/s. A split has to win by 10 %, and its partial tiles
+// to fit in `room` bytes.
+MidPlan plan_mid(int kind, int group, int64_t m, int64_t n, int64_t k, size_t room) {
   MidPlan best{0, 1, 0.0};
   if (m <= kSkinnyMaxRows || m > kMidMaxRows || n < 1 || k < kMidMinK) return best;
   struct Tile {
@@ -491,7 +492,9 @@ MidPlan plan_mid(int kind, int group, int64_t m, int64_t n, int64_t k) {
   const int count = kind == MID_I8 ? 1 : (kind == MID_W4 && group == 32) ? 2 : 3;
   const int64_t stages = (k + 127) / 128;
   for (int splits = 1; splits <= 8; splits *= 2) {
-    if (splits > 1 && (m > 1024 || stages < 4 * splits || splits * m * n * 4 > (int64_t(256) << 20))) break;
+    if (splits > 1 && (m > 1024 || stages < 4 * splits || splits * m * n * 4 > (int64_t(256) << 20) ||
+                       mid_partial_bytes(splits, m, n) > room))
+      break;
     for (int i = 0; i < count; ++i) {
       const int64_t per = (stages + splits - 1) / splits;
       if (kind == MID_W4 && tiles[i].ring_kb * 1024 + per * (128 / group) * 1024 > kMaxLds) continue;
@@ -504,11 +507,6 @@ MidPlan plan_mid(int kind, int group, int64_t m, int64_t n, int64_t k) {
     }
   }
   return best;
-}
-
-int64_t mid_w4_lds(int bm, int group, int64_t k) {
-  const int slots = bm == 32 || (bm == 64 && group == 128) ? 4 : 3;
-  return slots * (bm * 256 + 8192) + (k + 127) / 128 * (128 / group) * 1024;
 }
 
 hipError_t launch_mid_fp8(const MidArgs& p, int bm, bool f16a, bool e5, hipStream_t stream) {

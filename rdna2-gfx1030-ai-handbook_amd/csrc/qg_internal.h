@@ -259,9 +259,11 @@ struct MidPlan {
   int splits;
   double us;   // the model's time
 };
-MidPlan plan_mid(int kind, int group, int64_t m, int64_t n, int64_t k);
-// LDS bytes of an unsplit INT4 call.
-int64_t mid_w4_lds(int bm, int group, int64_t k);
+// Workspace of the partial tiles.
+inline size_t mid_partial_bytes(int64_t splits, int64_t m, int64_t n) {
+  return splits > 1 ? static_cast<size_t>((4 * splits * m * n + 255) / 256 * 256) : 0;
+}
+MidPlan plan_mid(int kind, int group, int64_t m, int64_t n, int64_t k, size_t room = SIZE_MAX);
 hipError_t launch_mid_fp8(const MidArgs& p, int bm, bool f16a, bool e5, hipStream_t stream);
 hipError_t launch_mid_i8(const MidArgs& p, hipStream_t stream);
 hipError_t launch_mid_w4(const W4Args& a, int bm, int splits, void* partial, hipStream_t stream);

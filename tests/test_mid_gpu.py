@@ -171,6 +171,35 @@ def test_int4_without_workspace(cuda):
     assert (out - ref).abs().max().item() <= 1e-4 * ref.abs().max().item()  # fp32 sums in another order
 
 
+@pytest.mark.parametrize("m,n,k,g,room,taken", [
+    (1000, 1024, 14336, 32, 2 * 1024 * 14336, True),   # 8 splits planned, which need more: dequant
+    (100, 4096, 4096, 32, 2 * 4096 * 4096, True), (100, 4096, 4096, 32, 0, False),
+    (300, 4096, 4096, 32, 1 << 20, False),             # parameters of K past LDS, no room to dequantize
+    (200, 1000, 1536, 32, 0, True), (300, 8192, 4096, 64, 0, True),  # unsplit
+    (300, 8192, 8192, 64, 2 * 8192 * 8192, True), (300, 8192, 8192, 64, 0, False),
+    (40, 300, 8192, 64, 0, True), (1024, 4096, 8192, 64, 2 * 4096 * 8192, True),
+])
+def test_int4_with_less_workspace(cuda, m, n, k, g, room, taken):
+    """Less workspace than the query reports: the dequant formulation's 2 n k
+    bytes always suffice, without them the call runs unsplit where it can."""
+    from rdna2_ops import _lib
+    from rdna2_ops import int4_weight_gemm_v07 as w4
+    case(f"mid int4 {m}x{n}x{k} g{g} room {room}")
+    gen = torch.Generator().manual_seed(m + n + k + g)
+    p = w4.pack_int4((torch.randn(n, k, generator=gen) * 0.02).to(cuda), group_size=g)
+    a = torch.randn(m, k, generator=gen).to(torch.bfloat16).to(cuda)
+    lib, P = _lib.library(), _lib.ptr
+    ws = torch.empty(max(room, 256), dtype=torch.uint8, device=cuda)
+    out = torch.empty(m, n, device=cuda)
+    status = lib.qg_w4a16_gemm(P(a), _lib.BF16, k, m, k, P(p.data), n, g, p.flags, P(p.scales), _lib.F32, P(p.zeros),
+                               None, 0, P(out), _lib.F32, P(ws) if room else None, room, _lib.stream_of(a))
+    assert (status == 0) == taken, status
+    if taken:
+        ref = a.double() @ w4.unpack_int4(p, dtype=torch.float32).double().T
+        # weights rounded to bf16 at worst: 2^-9 of each product, so of their root sum of squares
+        assert (out - ref).norm() <= 2.0 ** -8 * ref.norm()
+
+
 @pytest.mark.parametrize("m,n,k", [(17, 140, 6160), (64, 300, 12288), (65, 1000, 4096), (130, 257, 6160),
                                    (256, 3072, 8192), (300, 513, 8192)])
 def test_int8_split_shapes(cuda, m, n, k):
