@@ -587,15 +587,29 @@ double skinny_w4_us(int64_t m, int64_t n, int64_t k, int group_size) {
   return 1.5 + ((n + 15) / 16 + 255) / 256 * ((k + 127) / 128) * stage;
 }
 
+// Model time (us) of the tiled kernel (k_wd_gemm, past 64 rows, K a multiple of
+// 128): a stage of 128 K elements takes 1.4 us up to 128 tiles of 128 x 128
+// (which run as 128 x 64), 1.8 to 2.2 us in one round of 256 and 1.8 us for
+// each further round; group 64 1.4 and 1.65 times that. Measured, group 128:
+// 512 x 1024 x 8192 91 us, 1536 x 1536 x 6144 96, 1024 x 4096 x 8192 147, 1024
+// x 4096 x 11008 172, 1026 x 4096 x 11008 325, 2048 x 3072 x 12288 402; group
+// 64: 300 x 4096 x 8192 128.
+double tiled_w4_us(int64_t m, int64_t n, int64_t k, int group_size) {
+  const int64_t tiles = ((m + 127) / 128) * ((n + 127) / 128), rounds = (tiles + 255) / 256;
+  const double stage = tiles <= 128 ? 1.4 : 1.8 + (rounds > 1 ? 0.4 : 0.4 * tiles / 256) + 1.8 * (rounds - 1);
+  return 4.5 + (k / 128) * stage * (group_size == 128 ? 1.0 : tiles <= 128 ? 1.4 : 1.65);
+}
+
 // The kernel of a W4A16 call past 16 rows in the nk layout with K >= 1024:
-// mid_gemm where its model beats, by 10 %, the kernel that served the call
-// before it: k_w4_skinny up to 64 rows, the dequant formulation where
-// w4_prefill_bytes asks for it (the unpack's bytes at 4.4 TB/s, then the
-// ping-pong GEMM), and in any case the tiled kernel (N 4096, K 4096, M 512,
-// group 128: 48 -> 36 us; group 64, M 333: 66 -> 44 us; N 3072, K 12288, M 512:
-// 129 -> 88 us). Calls that multiplied exact group sums still do: none moves to
-// the dequant formulation, which rounds the weights. kn layout and shorter K:
-// as w4_prefill_bytes says.
+// mid_gemm where its model beats, by 10 %, k_w4_skinny (up to 64 rows) or the
+// dequant formulation where w4_prefill_bytes asks for it (the unpack's bytes at
+// 4.4 TB/s, then the ping-pong GEMM), and where it is not above the tiled
+// kernel's elsewhere (N 4096, K 4096, M 512, group 128: 48 -> 36 us; group 64,
+// M 333: 66 -> 44 us; N 3072, K 12288, M 512: 129 -> 88 us; but past 1024 rows
+// of a K whose parameters leave only 32-row tiles N 4096, K 11008, M 2048: 335
+// us tiled, 495 here). Calls that multiplied exact group sums still do: none
+// moves to the dequant formulation, which rounds the weights. kn layout and
+// shorter K: as w4_prefill_bytes says.
 struct W4Plan {
   qg::MidPlan mid;       // bm > 0: mid_gemm
   size_t dequant_bytes;  // > 0: dequant + ping-pong
@@ -610,11 +624,13 @@ W4Plan plan_w4(int64_t m, int64_t n, int64_t k, int group_size, int flags, size_
   W4Plan pl{qg::MidPlan{0, 1, 0.0}, w4_prefill_bytes(m, n, k, group_size)};
   if ((flags & QG_W4_LAYOUT_KN) || m <= qg::kSkinnyMaxRows || k < qg::kMidMinK) return pl;
   pl.mid = qg::plan_mid(qg::MID_W4, group_size, m, n, k, room);
-  double before_us = 1.0e9;
-  if (m <= kW4TiledMinRows) before_us = skinny_w4_us(m, n, k, group_size);
+  double bar_us = 1.0e9;
+  if (m <= kW4TiledMinRows) bar_us = 0.9 * skinny_w4_us(m, n, k, group_size);
   else if (pl.dequant_bytes > 0 && pl.dequant_bytes <= room)
-    before_us = 2.5 + n * k * 2.5 / 4.4e6 + pingpong_us(m, n, k);
-  if (pl.mid.us > 0.9 * before_us) pl.mid.bm = 0;
+    bar_us = 0.9 * (2.5 + n * k * 2.5 / 4.4e6 + pingpong_us(m, n, k));
+  else if (pl.dequant_bytes == 0 && k % kStageK == 0)
+    bar_us = tiled_w4_us(m, n, k, group_size);
+  if (pl.mid.us > bar_us) pl.mid.bm = 0;
   return pl;
 }
 
