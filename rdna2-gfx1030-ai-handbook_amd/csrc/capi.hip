@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -571,9 +572,8 @@ size_t w4_prefill_bytes(int64_t m, int64_t n, int64_t k, int group_size) {
   return static_cast<size_t>(round_up(2 * n * k, 256));
 }
 
-// Model time (us) of a ping-pong GEMM on 2-byte activations: rounds of 256
-// tiles of 256 x 192, 0.8 us per 64-element stage (M 2048, N = K = 3072, 128
-// tiles of fp8: 69 us with the 128-row tiles of k_wd_gemm, 45 us this way).
+// Model time (us) of a ping-pong GEMM on 2-byte operands: rounds of 256 tiles of
+// 256 x 192, 0.8 us per 64-element stage.
 double pingpong_us(int64_t m, int64_t n, int64_t k) {
   const int64_t tiles = ((m + 255) / 256) * ((n + 191) / 192);
   return 5.0 + (tiles + 255) / 256 * ((k + 63) / 64) * 0.8;
@@ -801,20 +801,45 @@ struct Fp8Plan {
   size_t total() const { return a_bytes + w_bytes + partial_bytes; }
 };
 
+// The kernel of a call past 16 rows with K >= 1024 and fewer than 192 tiles of
+// 256 x 192: the least of three models (us). Over 275 sizes (M 300 to 8192, N 64
+// to 6144, K 1024 to 12288) the choice is within 7 % of the fastest of the three.
+//  * the ping-pong GEMM, fp8 W converted in registers: one round of tiles, 0.88
+//    us per 64-element stage, and up to 17 us for the elementwise stores of a
+//    partial edge tile, by how much of the tile is filled (K 1024: N 3072, M 2048
+//    23.7 us, M 1500 40.5; M 4096, N 64 25.4). It has to win by 5 %;
+//  * the 128 x 128 tiles of k_wd_gemm: 1.55 us per 128-element stage in one
+//    round of 256 workgroups, 2.6 to 3 us past it (M 2049, N 64, K 1024 16.3 us,
+//    M 4096, N 768, K 12288 158, M 2048, N 3072, K 3072 70);
+//  * mid_gemm's model, and 10 us for the epilogues of several rounds (M 700, N
+//    6144, K 1024 32 us).
+enum Fp8Kernel { FP8_MID, FP8_TILED, FP8_PINGPONG };
+Fp8Kernel choose_fp8(const qg::MidPlan& mid, int64_t m, int64_t n, int64_t k) {
+  const double edge = std::max((m % 256) / 256.0, (n % 192) / 192.0);
+  const double pingpong = 5.5 + ((k + 63) / 64) * 0.88 + 17.0 * edge;
+  const int64_t tiles = ((m + 127) / 128) * ((n + 127) / 128);
+  const double stage = n <= 64 ? 1.3 : tiles <= 256 ? 1.55 : 2.2 + 0.4 * std::min(2.0, tiles / 256.0);
+  const double tiled = 6.0 + ((k + 127) / 128) * stage;
+  double split = 1.0e9;
+  if (mid.bm > 0) split = mid.us + (((m + mid.bm - 1) / mid.bm) * ((n + 127) / 128) * mid.splits > 256 ? 10.0 : 0.0);
+  if (pingpong < 0.95 * std::min(tiled, split)) return FP8_PINGPONG;
+  return split <= tiled ? FP8_MID : FP8_TILED;
+}
+
 Fp8Plan plan_fp8(const void* a, int64_t a_sm, int64_t a_sk, const void* w, int64_t w_sn, int64_t w_sk,
                  int64_t m, int64_t n, int64_t k) {
   Fp8Plan pl;
   pl.kp = round_up(k, kStageK);
   pl.skinny = m <= qg::kSkinnyMaxRows && k > 0;
   pl.mid = qg::plan_mid(qg::MID_FP8, 128, m, n, k);
-  // >= 192 tiles of 256 x 192 (the INT8 kernel's large-grid rule), or where the
-  // model puts it before mid_gemm's tiles: the ping-pong GEMM, fp8 W converted
-  // exactly to A's 2-byte type in registers
+  // from 192 tiles of 256 x 192 (the INT8 kernel's large-grid rule) always the
+  // ping-pong GEMM, fp8 W converted exactly to A's 2-byte type in registers
   const int64_t tiles = ((m + 255) / 256) * ((n + 191) / 192);
-  pl.pingpong = !pl.skinny && 2 * m * pl.kp < kMaxOperandBytes &&
-                (tiles >= 192 || (m > qg::kSkinnyMaxRows && k >= qg::kMidMinK &&
-                                  (pl.mid.bm == 0 || pingpong_us(m, n, k) < 0.9 * pl.mid.us)));
-  if (pl.pingpong) pl.mid.bm = 0;
+  Fp8Kernel kernel = FP8_TILED;
+  if (tiles >= 192) kernel = FP8_PINGPONG;
+  else if (m > qg::kSkinnyMaxRows && k >= qg::kMidMinK) kernel = choose_fp8(pl.mid, m, n, k);
+  pl.pingpong = kernel == FP8_PINGPONG && !pl.skinny && 2 * m * pl.kp < kMaxOperandBytes;
+  if (kernel != FP8_MID) pl.mid.bm = 0;
   // the streaming kernels take whole 16-byte chunks of a row, the tiled ones whole stages
   const int64_t whole = pl.skinny || pl.mid.bm > 0 ? 16 : kStageK;
   pl.ks = k % whole == 0 ? k : pl.kp;

@@ -236,6 +236,20 @@ def test_w4a16_choice_of_many_rows_and_long_k(lib, m, n, k, mid):
     assert (choice > _lib.CHOICE_PINGPONG) == mid and (mid or choice == 0), choice
 
 
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (2049, 64, 1024, "tiled"), (4096, 128, 3072, "tiled"), (8192, 64, 12288, "tiled"), (4096, 768, 12288, "tiled"),
+    (1500, 3072, 1024, "tiled"), (700, 6144, 1024, "tiled"),
+    (2048, 3072, 3072, "pingpong"), (4096, 1536, 1024, "pingpong"), (1500, 4096, 12288, "pingpong"),
+    (4096, 12288, 128, "pingpong"),
+    (17, 3072, 3072, "mid"), (1024, 768, 3072, "mid"), (2048, 768, 12288, "mid"), (2048, 64, 1024, "mid"),
+])
+def test_fp8_choice_of_smaller_grids(lib, m, n, k, kernel):
+    """fp8 weights below 192 tiles of 256 x 192: the fastest measured of the
+    tiled, the ping-pong and the multi-stage kernel."""
+    choice = lib.qg_row_kernel_choice(_lib.CHOICE_FP8, 0, 0, m, n, k)
+    assert kernel == {0: "tiled", _lib.CHOICE_PINGPONG: "pingpong"}.get(choice, "mid"), choice
+
+
 def test_moe_dispatch_qx_rejects_invalid_arguments(lib):
     """The fused routing + x quantization takes bf16 rows of at most 2048
     values, a multiple of 8, 16-byte aligned x and 8-byte aligned xq rows;
