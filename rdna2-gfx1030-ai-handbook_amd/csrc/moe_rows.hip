@@ -9,10 +9,13 @@
 // chunks w, w + 4, ... into a ring of its own (no barrier until the partial
 // tiles are summed, as in k_skinny_gemm), and three workgroups per CU overlap
 // one another's table reads, copies and epilogues. Up to 8 rows copy half of
-// the activation bytes that up to 16 do; more rows of an entry repeat the walk
-// over its weights. 16 tokens, 64 experts, top-8, hidden 2048, inter 768 (56 of
-// the experts in use): gate/up 176 MB 50.5 -> 31.3 us (5.6 TB/s), down 88 MB
-// 32.7 -> 20.0 us (4.4 TB/s).
+// the activation bytes that up to 16 do. An entry of more rows (a skewed router)
+// takes 64 at a time, 16 a wave, all waves on one chunk of the weights: passes of
+// 16 rows over the weights instead cost 162.9 us at 64 tokens on the same 8 of 64
+// experts, hidden 4096, inter 2048, where the tiles take 98.6 and this 75. 16
+// tokens, 64 experts, top-8, hidden 2048, inter 768 (56 of the experts in use):
+// gate/up 176 MB 50.5 -> 31.3 us (5.6 TB/s), down 88 MB 32.7 -> 20.0 us (4.4
+// TB/s).
 #include "qg_common.h"
 #include "qg_epilogue.h"
 #include "qg_internal.h"
@@ -23,6 +26,7 @@ namespace qg {
 namespace {
 
 constexpr int kMoeRowsWaves = 4, kMoeRowsDepth = 2, kMoeRowsCT = 2;
+constexpr int kMoeTallSlots = 4;  // ring of the tall form
 
 template <int RP_, int CT_>
 struct MoeRowsCfg {
@@ -43,42 +47,53 @@ struct MoeRowsTile {
   int n0;
 };
 
-// Rows [t.first, t.stop), RP at a time, of one table entry and column block.
-template <int MOE, int RP, int CT>
+// Rows [t.first, t.stop) of one table entry and column block, RP at a time, the
+// K chunks spread over the waves. TALL (entries of many rows): 16 rows a wave
+// and all waves on the same chunk, in a ring of kMoeTallSlots chunks that they
+// fill together, one barrier per chunk; the weights are copied once for 64 rows.
+template <int MOE, int RP, int CT, bool TALL>
 __device__ __forceinline__ void moe_rows_body(const I8GemmArgs& p, const MoeRowsTile& t, char* smem) {
 #pragma clang fp contract(off)
   using C = MoeRowsCfg<RP, CT>;
   constexpr int NW = C::NW, D = C::D;
+  constexpr int PASS = TALL ? 16 * NW : RP;  // rows per pass
+  // copies of a wave and chunk, 8 rows of 128 bytes each
+  constexpr int A_COPIES = TALL ? PASS / 8 / NW : C::A_COPIES, W_COPIES = TALL ? 2 * CT / NW : C::W_COPIES;
+  constexpr int STAGE = TALL ? (PASS + 16 * CT) * C::KS : C::STAGE, W_AT = PASS * C::KS;
+  static_assert(!TALL || (2 * CT % NW == 0 && kMoeTallSlots * STAGE <= C::RING), "copies and ring of the tall form");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, q = lane >> 4;
-  char* const ring = smem + wave * D * C::STAGE;
+  char* const ring = TALL ? smem : smem + wave * D * STAGE;
   const uint32_t ring_addr = lds_addr_of(ring);
   const int slot16 = lane & 7;  // 16-byte slot of a lane in its 128-byte LDS row
+  const int row8 = lane >> 3;   // row of a lane in a copy
+  // copy i of a wave: rows 8 copy_of(i) .. + 7 of the operand
+  auto copy_of = [&](int i) __attribute__((always_inline)) { return TALL ? wave + NW * i : i; };
   auto source = [&](int row) __attribute__((always_inline)) {
     return min(max(p.row_token ? p.row_token[row] : row, 0), p.a_rows - 1);
   };
 
-  uint32_t woff[C::W_COPIES];
-  static_for<0, C::W_COPIES>([&](auto i) {
-    const int c = 8 * i + (lane >> 3);
+  uint32_t woff[W_COPIES];
+  static_for<0, W_COPIES>([&](auto i) {
+    const int c = 8 * copy_of(i) + row8;
     woff[i] = static_cast<uint32_t>(min(t.n0 + c, p.N - 1)) * static_cast<uint32_t>(p.w_sn) +
               16u * (slot16 ^ lds_row_xor<C::KS>(c & 15));
   });
   const int chunks = p.K / C::KS;
-  const int n = chunks > wave ? (chunks - wave + NW - 1) / NW : 0;
+  const int n = TALL ? chunks : chunks > wave ? (chunks - wave + NW - 1) / NW : 0;
 
-  for (int r0 = t.first; r0 < t.stop; r0 += RP) {
+  for (int r0 = t.first; r0 < t.stop; r0 += PASS) {
     // everything that is read through registers is requested before the copies
-    uint32_t aoff[C::A_COPIES];
-    static_for<0, C::A_COPIES>([&](auto i) {
-      const int r = 8 * i + (lane >> 3);
+    uint32_t aoff[A_COPIES];
+    static_for<0, A_COPIES>([&](auto i) {
+      const int r = 8 * copy_of(i) + row8;
       aoff[i] = static_cast<uint32_t>(source(min(r0 + r, t.stop - 1))) * static_cast<uint32_t>(p.a_sm) +
-                16u * (slot16 ^ lds_row_xor<C::KS>(r));
+                16u * (slot16 ^ lds_row_xor<C::KS>(r & 15));
     });
     // output elements of this thread: (row, column), or (row, feature) for SiLU * mul
     constexpr int OC = MOE == QG_MOE_EPI_SILU_MUL ? 8 * CT : 16 * CT;
-    constexpr int PER = (RP * OC + 64 * NW - 1) / (64 * NW);
+    constexpr int PER = (PASS * OC + 64 * NW - 1) / (64 * NW);
     float sa[PER], sb[PER], sb2[PER], rw[PER];
     int dst[PER], at[PER];
     static_for<0, PER>([&](auto i) {
@@ -87,7 +102,7 @@ __device__ __forceinline__ void moe_rows_body(const I8GemmArgs& p, const MoeRows
       // gate column of feature oc; its up column is 16 further on
       const int cc = MOE == QG_MOE_EPI_SILU_MUL ? 32 * (oc >> 4) + (oc & 15) : oc;
       const int row = r0 + rr;
-      const bool in = rr < RP && row < t.stop && t.n0 + cc < p.N;
+      const bool in = rr < PASS && row < t.stop && t.n0 + cc < p.N;
       at[i] = rr * C::PITCH + cc;
       dst[i] = in ? row : -1;
       sa[i] = sb[i] = sb2[i] = rw[i] = 0.0f;
@@ -105,34 +120,57 @@ __device__ __forceinline__ void moe_rows_body(const I8GemmArgs& p, const MoeRows
     });
 
     auto issue = [&](int c, int slot) __attribute__((always_inline)) {
-      const uint32_t to = ring_addr + slot * C::STAGE;
-      static_for<0, C::W_COPIES>([&](auto i) {
-        dma16s_nt(t.w, woff[i] + static_cast<uint32_t>(C::KS * c), to + C::W_AT + 1024 * i);
+      const uint32_t to = ring_addr + slot * STAGE;
+      static_for<0, W_COPIES>([&](auto i) {
+        if constexpr (TALL) dma16s(t.w, woff[i] + static_cast<uint32_t>(C::KS * c), to + W_AT + 1024 * copy_of(i));
+        else dma16s_nt(t.w, woff[i] + static_cast<uint32_t>(C::KS * c), to + W_AT + 1024 * i);
       });
-      static_for<0, C::A_COPIES>([&](auto i) {
-        dma16s(p.a, aoff[i] + static_cast<uint32_t>(C::KS * c), to + 1024 * i);
+      static_for<0, A_COPIES>([&](auto i) {
+        dma16s(p.a, aoff[i] + static_cast<uint32_t>(C::KS * c), to + 1024 * copy_of(i));
       });
     };
     i32x4 acc[CT];
     static_for<0, CT>([&](auto j) { acc[j] = i32x4{0, 0, 0, 0}; });
-    static_for<0, D>([&](auto d) {
-      if (d < n) issue(wave + NW * d, d);
-    });
-    const int arow = min(col, RP - 1);
-    for (int i = 0; i < n; ++i) {
-      if (i + 1 < n) wait_vm<C::COPIES>();
-      else wait_vm<0>();
-      const char* const st = ring + (i & 1) * C::STAGE;
+    const int arow = TALL ? 16 * wave + col : min(col, RP - 1);
+    auto product = [&](int slot) __attribute__((always_inline)) {
+      const char* const st = ring + slot * STAGE;
       static_for<0, 2>([&](auto u) {
-        const i32x4 a = *reinterpret_cast<const i32x4*>(st + arow * C::KS + 16 * ((4 * u + q) ^ lds_row_xor<C::KS>(arow)));
+        const i32x4 a = *reinterpret_cast<const i32x4*>(st + arow * C::KS +
+                                                        16 * ((4 * u + q) ^ lds_row_xor<C::KS>(arow & 15)));
         static_for<0, CT>([&](auto j) {
-          const i32x4 w = *reinterpret_cast<const i32x4*>(st + C::W_AT + (16 * j + col) * C::KS +
+          const i32x4 w = *reinterpret_cast<const i32x4*>(st + W_AT + (16 * j + col) * C::KS +
                                                           16 * ((4 * u + q) ^ lds_row_xor<C::KS>(col)));
           acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, w, acc[j], 0, 0, 0);
         });
       });
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot's reads are done
-      if (i + D < n) issue(wave + NW * (i + D), i & 1);
+    };
+    if constexpr (TALL) {
+      // top of chunk i: it has landed everywhere and every wave has read chunk
+      // i - 1, whose slot takes chunk i + R - 1
+      constexpr int R = kMoeTallSlots, COPIES = A_COPIES + W_COPIES;
+      static_assert(R == 4, "waits below");
+      static_for<0, R - 1>([&](auto d) {
+        if (d < n) issue(d, d);
+      });
+      for (int i = 0; i < n; ++i) {
+        const int after = n - 1 - i;  // chunks issued after this one: min(after, R - 2)
+        if (after >= 2) wait_vm_barrier<2 * COPIES>();
+        else if (after == 1) wait_vm_barrier<COPIES>();
+        else wait_vm_barrier<0>();
+        if (i + R - 1 < n) issue(i + R - 1, (i + R - 1) % R);
+        product(i % R);
+      }
+    } else {
+      static_for<0, D>([&](auto d) {
+        if (d < n) issue(wave + NW * d, d);
+      });
+      for (int i = 0; i < n; ++i) {
+        if (i + 1 < n) wait_vm<C::COPIES>();
+        else wait_vm<0>();
+        product(i & 1);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot's reads are done
+        if (i + D < n) issue(wave + NW * (i + D), i & 1);
+      }
     }
 
     int* const red = reinterpret_cast<int*>(smem);
@@ -147,8 +185,10 @@ __device__ __forceinline__ void moe_rows_body(const I8GemmArgs& p, const MoeRows
       if (dst[i] < 0 || dst[i] >= p.out_rows) return;
       auto sum = [&](int word) __attribute__((always_inline)) {
         int v = red[word];
+        if constexpr (!TALL) {
 #pragma unroll
-        for (int w = 1; w < NW; ++w) v += red[w * 16 * C::PITCH + word];
+          for (int w = 1; w < NW; ++w) v += red[w * 16 * C::PITCH + word];
+        }
         return v;
       };
       const int e = threadIdx.x + 64 * NW * i;
@@ -166,7 +206,7 @@ __device__ __forceinline__ void moe_rows_body(const I8GemmArgs& p, const MoeRows
         static_cast<uint16_t*>(p.out)[o] = f32_to_bf16(y * rw[i]);
       }
     });
-    if (r0 + RP < t.stop) __syncthreads();  // the partial tiles have been read
+    if (r0 + PASS < t.stop) __syncthreads();  // the partial tiles have been read
   }
 }
 
@@ -182,8 +222,10 @@ __global__ __launch_bounds__(64 * kMoeRowsWaves) void k_moe_rows(I8GemmArgs p) {
   if (e < 0 || e >= p.n_experts || m0 < 0 || m0 >= p.M || m_end <= m0 || m_end > p.M) return;
   const MoeRowsTile t{p.w + e * p.w_estride, p.b_scale ? p.b_scale + static_cast<int64_t>(e) * p.N : nullptr, m0,
                       min(m_end, m0 + QG_MOE_TILE_ROWS), (static_cast<int>(blockIdx.x) - tile * cols) * 16 * CT};
-  if (t.stop - t.first <= 8) moe_rows_body<MOE, 8, CT>(p, t, smem);
-  else moe_rows_body<MOE, 16, CT>(p, t, smem);
+  const int rows = t.stop - t.first;
+  if (rows <= 8) moe_rows_body<MOE, 8, CT, false>(p, t, smem);
+  else if (rows <= 16) moe_rows_body<MOE, 16, CT, false>(p, t, smem);
+  else moe_rows_body<MOE, 16, CT, true>(p, t, smem);
 }
 
 template <int MOE>
@@ -197,19 +239,19 @@ hipError_t launch_moe_rows_e(const I8GemmArgs& p, hipStream_t stream) {
 }  // namespace
 
 // Few rows per expert. A gathered operand of up to 32 tokens (a token takes an
-// expert at most once, so up to two passes), or of up to 64 where rows_max
-// leaves 16 rows per expert on average after the dispatch's default padding to
-// 64 (with another padding at most four passes); up to 16 slots per expert
-// behind the route epilogue. Whole MoE calls against the persistent tiles (us):
-//   tokens, experts, top-k, hidden, inter    tiles   here
-//   16, 64, 8, 2048, 768                     104.0   67.8   2 rows an expert
-//   64, 64, 8, 2048, 768                     105.9   77.4   8
-//   16, 8, 8, 2048, 1024                      59.6   34.8   16
-//   32, 16, 8, 3072, 1024                     78.6   64.7   16
-//   32, 8, 8, 2048, 1024                      59.7   49.4   32, gate/up here only
-//   64, 16, 8, 3072, 1024                     79.3   83.0   32, gate/up here only
-//   64, 8, 8, 2048, 1024                      59.4   58.8   64, gate/up here only
-//   1000, 64, 1, 1024, 512                    58.6   57.8   16, down here only
+// expert at most once), or of up to 64 where rows_max leaves 16 rows per expert
+// on average after the dispatch's default padding to 64; up to 16 slots per
+// expert behind the route epilogue, however the router spreads them (the tall
+// form keeps even all tokens on the same experts within 4 % of the tiles).
+// Whole MoE calls against the persistent tiles (us, tiles / here):
+//   tokens, experts, top-k, hidden, inter    even routing     the same experts
+//   16, 64, 8, 2048, 768                     104.5    66.7     59.8    32.8
+//   64, 64, 8, 2048, 768                     104.8    78.5     59.7    37.5
+//   32, 16, 8, 4096, 2048                    121.2    94.6     91.4    64.4
+//   64, 8, 2, 2048, 768                       56.4    33.4     56.8    30.5
+//   128, 64, 8, 4096, 2048 (down here only)  387.3   367.4    100.7   104.3
+//   512, 64, 1, 2048, 768 (down here only)   103.3    93.2     59.5    56.0
+//   1000, 64, 1, 2048, 768 (down here only)  114.3   103.9     63.0    61.3
 bool moe_rows_applies(const I8GemmArgs& p) {
   const int64_t few = static_cast<int64_t>(kMoeFewRows) * p.n_experts;
   if (p.moe_epi == QG_MOE_EPI_ROUTE) return p.out_rows <= few;

@@ -395,6 +395,20 @@ def test_moe_few_rows_skewed(cuda):
     run_and_check(cuda, x, logits, wg, wu, wd, 2, label="few rows skewed")
 
 
+# entries of more than 16 rows (a skewed router): 64 rows a pass, 16 a wave; one
+# to five K chunks through the ring of four, whole and partial passes, up to 192
+# rows of an entry (the gate/up product takes them up to 64 tokens, the down
+# product up to 16 slots per expert)
+@pytest.mark.parametrize("t,e,h,f,top_k", [(17, 8, 128, 256, 1), (33, 8, 256, 384, 2), (48, 16, 384, 128, 1),
+                                           (63, 16, 512, 640, 2), (64, 8, 640, 512, 1), (65, 16, 256, 384, 1),
+                                           (129, 16, 384, 128, 1), (192, 16, 128, 640, 1), (200, 64, 256, 256, 2)])
+def test_moe_few_rows_same_experts(cuda, t, e, h, f, top_k):
+    case(f"moe few rows, same experts t{t} e{e} h{h} f{f} k{top_k}")
+    x, logits, wg, wu, wd = make_case(300 + t, t, e, h, f, top_k)
+    logits[:, 1:1 + top_k] += 20.0
+    run_and_check(cuda, x, logits, wg, wu, wd, top_k, label=f"same experts t{t}")
+
+
 @pytest.mark.parametrize("n", [32, 96, 77])
 def test_moe_few_rows_table_and_edges(cuda, n):
     """Entries that name no expert, one past the last, or rows outside the
