@@ -388,8 +388,9 @@ int qg_moe_sizes(int64_t tokens, int n_experts, int top_k, int pad, int64_t* row
  * expert's valid rows, 0}; tiles[0][3] = number of tiles in use (the used
  * tiles come first). counts: int32 workspace [QG_MOE_COUNTS_PER_EXPERT *
  * n_experts]: per-expert counts, segment offsets and first tiles, then the
- * sort's per-block histograms. Two launches, no host synchronisation and no
- * memset (capturable in a graph). */
+ * histograms of the sort's blocks (ceil(tokens / tb) rows of n_experts, tb =
+ * ceil(tokens / 256) tokens a block). One launch up to 16 tokens, else two; no
+ * host synchronisation and no memset (capturable in a graph). */
 int qg_moe_dispatch(const float* logits, int64_t l_sm, int64_t tokens, int n_experts, int top_k, int pad,
                     int32_t* experts, float* weights, int32_t* counts, int32_t* row_token,
                     float* row_weight, int32_t* row_slot, int64_t rows_max, int32_t* tiles,

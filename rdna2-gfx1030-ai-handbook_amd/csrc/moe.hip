@@ -1,6 +1,7 @@
 // MoE prefill routing, dispatch and combine on gfx950 (benchmark configuration
 // 4; the reference repository has no MoE kernel). The grouped INT8 GEMM that
-// runs between dispatch and combine is k_i8_moe_pp in int8_gemm.hip.
+// runs between dispatch and combine is k_i8_moe_pp in int8_gemm.hip, with few
+// rows per expert k_moe_rows in moe_rows.hip.
 //
 // The dispatch is a stable counting sort of the tokens * top_k routed slots
 // by expert, in one launch up to kRouteWaves tokens (k_moe_dispatch_few), else
@@ -21,6 +22,9 @@
 //            rank among equal experts of its 64-slot step (six ballots). Rows
 //            inside a segment are in slot order: the dispatch is deterministic
 //   combine  out[t] = bf16(sum over k of y[t * top_k + k]) in k order (fp32)
+// counts layout: [0, E) counts, [E, 2E) segment offsets, [2E, 3E) first tile of
+// each expert, then [kMaxSortBlocks][E] per-block histograms (the workspace
+// holds (3 + 256) E ints; the blocks in use are written).
 #include "qg_common.h"
 #include "qg_internal.h"
 #include "qg_quant.h"
@@ -55,15 +59,11 @@ __device__ __forceinline__ int wave_inclusive_scan(int v) {
   return v;
 }
 
-// counts layout: [0, E) counts, [E, 2E) segment offsets, [2E, 3E) first tile
-// of each expert, then [kMaxSortBlocks][E] per-block histograms (the
-// workspace holds (3 + 256) E ints).
-// QX: the wave also quantizes token t's row of x (the per-token activation
-// quantization of the gate/up GEMM, bit-identical to k_quant_rows_reg): its
-// loads are issued before the routing, which they overlap, and the codes are
-// formed and stored after it.
 // One wave routes token t (lane = expert); chosen(e) is called by the lane of
-// each expert taken.
+// each expert taken. QX: the wave also quantizes token t's row of x (the
+// per-token activation quantization of the gate/up GEMM, bit-identical to
+// k_quant_rows_reg): its loads are issued before the routing, which they
+// overlap, and the codes are formed and stored after it.
 template <bool QX, typename F>
 __device__ __forceinline__ void route_token(const MoeDispatchArgs& p, int t, F&& chosen) {
 #pragma clang fp contract(off)
@@ -209,6 +209,8 @@ __global__ __launch_bounds__(kRouteWaves * 64) void k_moe_dispatch_few(MoeDispat
     td[2] = 0;
     td[3] = ti == 0 ? tiles_used : 0;
   }
+  // the histogram of each sort block, one token here
+  if (t < p.T && lane < p.E) p.counts[(3 + t) * p.E + lane] = takes[lane] >> t & 1;
   // slots of token t: the experts and weights that its own wave has stored
   if (t < p.T && lane < p.top_k) {
     const int s = t * p.top_k + lane;

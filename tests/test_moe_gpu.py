@@ -500,3 +500,19 @@ def test_moe_dispatch_few_tokens(cuda, t, e, k, pad):
     tl = it["tiles"].cpu().numpy()
     assert tl[0, 3] == len(want) and np.array_equal(tl[:len(want), :3], np.array(want))
     assert (tl[len(want):, 0] == -1).all() and (tl[1:, 3] == 0).all()
+
+
+@pytest.mark.parametrize("t,e,k", [(1, 8, 2), (5, 64, 8), (16, 33, 4), (17, 64, 8), (300, 16, 2)])
+def test_moe_dispatch_histograms(cuda, t, e, k):
+    """counts past 3 E: slots per expert of each sort block (ceil(t / 256)
+    tokens), whichever launches the dispatch takes."""
+    case(f"moe dispatch histograms t{t} e{e} k{k}")
+    logits = torch.randn(t, e, generator=torch.Generator().manual_seed(t + e))
+    m = mod()
+    x, _, wg, wu, wd = make_case(3, t, e, 128, 128, k)
+    prep = m.prepare_moe_weights(wg.to(cuda), wu.to(cuda), wd.to(cuda))
+    _, it = m.moe_int8_forward(x.to(cuda), logits.to(cuda), prep, top_k=k, return_intermediates=True)
+    tb = -(-t // 256)
+    want = np.zeros((-(-t // tb), e), np.int32)
+    np.add.at(want, (np.repeat(np.arange(t) // tb, k), it["experts"].cpu().numpy().reshape(-1)), 1)
+    assert np.array_equal(it["counts"].cpu().numpy()[3 * e:3 * e + want.size].reshape(want.shape), want)
