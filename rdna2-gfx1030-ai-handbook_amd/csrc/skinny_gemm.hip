@@ -356,19 +356,14 @@ hipError_t launch_skinny_fp8_rows(const SkinnyArgs& p, hipStream_t stream) {
 }
 
 // INT4 column tiles: four pay only at 16 rows (uint4, N 14336, K 4096: 19 / 14
-// / 17 / 12 us with 1 / 2 / 3 / 4), one or two below; up to K 512, where half
-// of the waves have no chunk and every choice takes 3 to 4 us, as many as the
-// registers of a wide workgroup allow. The parameters of K / G groups have to
-// fit next to the rings.
+// / 17 / 12 us with 1 / 2 / 3 / 4), one or two below. The same rule holds for a
+// short K (16 rows, N 14336, K 256: group 32 7.8 us against 10.5 with one tile,
+// group 64, N 28672, K 512 10.1 against 12.5 with two). The parameters of K / G
+// groups have to fit next to the rings.
 template <typename C1>
 int skinny_w4_tiles(const SkinnyArgs& p) {
-  int ct;
-  if (p.K <= 512) {
-    ct = C1::RP == 4 ? 2 : C1::G == 128 ? 4 : C1::G == 64 ? 2 : 1;
-  } else {
-    const int allowed[] = {1, 2, 4};
-    ct = skinny_tiles(p.N, C1::A_COPIES, C1::W_COPIES, C1::RP == 16 && C1::G != 32 ? 4 : 2, allowed, 3);
-  }
+  const int allowed[] = {1, 2, 4};
+  int ct = skinny_tiles(p.N, C1::A_COPIES, C1::W_COPIES, C1::RP == 16 && C1::G != 32 ? 4 : 2, allowed, 3);
   while (ct > 1 && C1::RP * 4096 + ct * 16384 + skinny_par_bytes(p, 16 * ct) > kMaxLds) ct >>= 1;
   return ct;
 }
@@ -378,7 +373,7 @@ hipError_t launch_skinny_w4_rows(const SkinnyArgs& p, hipStream_t stream) {
   using C1 = SkinnyCfg<FMT, F16A, RP, 1, 2, G>;
   const int ct = skinny_w4_tiles<C1>(p);
   if (C1::PAR_AT + skinny_par_bytes(p, 16) > kMaxLds) return hipErrorInvalidValue;
-  if constexpr (RP > 4 && G != 32) {
+  if constexpr (RP == 16 && G != 32) {
     if (ct == 4) return launch_skinny_c<SkinnyCfg<FMT, F16A, RP, 4, 2, G>>(p, stream);
   }
   if (ct == 2) return launch_skinny_c<SkinnyCfg<FMT, F16A, RP, 2, 2, G>>(p, stream);

@@ -942,7 +942,7 @@ hipError_t launch_decode_kn(const W4Args& p, hipStream_t stream) {
   }
 }
 
-// uint4 storage whose 8 waves take exactly 4 chunks each (K 3585 .. 4096): the
+// uint4 storage whose 8 waves take up to 4 chunks each (K 3584 and 4096): the
 // decode kernel with all loads up front, against the streaming kernel of
 // skinny_gemm.hip, at K 4096 (us, both rotated weight copies, one box):
 //   N      M 4            M 8             M 16

@@ -402,10 +402,7 @@ def int4_linear_a16(a, p, *, bias=None, method="dequant", prepared=None, tile=(6
                                                  "k_w4_decodeILi{}ELi{}ELi128E".format(rp, ct))
             if _skinny_par_bytes(p, 16) <= 80 * 1024:
                 rp = 4 if m <= 4 else 8 if m <= 8 else 16
-                if p.k <= 512:
-                    ct = 2 if rp == 4 else {128: 4, 64: 2, 32: 1}[p.group_size]
-                else:
-                    ct = _lib.skinny_tiles(p.n, rp // 4, 1, (1, 2, 4) if rp == 16 and p.group_size != 32 else (1, 2))
+                ct = _lib.skinny_tiles(p.n, rp // 4, 1, (1, 2, 4) if rp == 16 and p.group_size != 32 else (1, 2))
                 while ct > 1 and 4096 * rp + 16384 * ct + _skinny_par_bytes(p, 16 * ct) > 160 * 1024:
                     ct //= 2
                 return out, _lib.kernel_metadata(

@@ -271,17 +271,31 @@ def test_uint4_multi_row_decode(cuda, m, n, k):
 
 
 def test_decode_metadata_column_tiles(cuda):
-    """The decode kernel's reported column tile follows the launcher's choice
-    per group size and row count (16 * CT columns)."""
+    """The reported column tile follows the launcher's choice (16 * CT columns)
+    and its instantiation exists. Streaming kernel: the fewest copies a CU, one
+    tile while a round of 256 workgroups holds the columns, up to two (four at 16
+    rows, groups 64 and 128) past it. uint4 whose waves take four chunks each:
+    the decode kernel from 8192 columns (2 to 4 rows) or 12288 (more)."""
     case("decode metadata column tiles")
     g = torch.Generator().manual_seed(9)
-    for group, m, cols in ((32, 1, 32), (32, 5, 16), (64, 5, 32), (128, 5, 64), (128, 3, 32)):
-        w = torch.randn(96, 512, generator=g) * 0.02
+    sizes = [(group, m, 96, k, 16) for group, m in ((32, 1), (32, 5), (64, 5), (128, 5), (128, 3)) for k in (512, 2048)]
+    sizes += [(64, 16, 4096, 640, 16), (64, 16, 4112, 640, 32), (64, 16, 8208, 640, 64), (32, 16, 8208, 640, 32),
+              (128, 16, 8208, 256, 64), (128, 8, 8208, 640, 32), (64, 4, 4112, 640, 32)]
+    for group, m, n, k, cols in sizes:
+        w = torch.randn(n, k, generator=g) * 0.02
         p = w4().pack_int4(w.to(cuda), group_size=group, symmetric=False)
-        a = torch.randn(m, 512, generator=g).to(torch.float16).to(cuda)
+        a = torch.randn(m, k, generator=g).to(torch.float16).to(cuda)
         _, md = w4().int4_linear_a16(a, p, method="dot2", return_kernel=True)
-        assert md["variant"] == "w4a16_decode" and md["tile"][1] == cols, (group, m, md)
-        assert md["vgpr"] is not None, (group, m)
+        assert md["variant"] == "w4a16_decode" and md["tile"][1] == cols, (group, m, n, k, md)
+        assert md["vgpr"] is not None and "k_skinny_gemm" in md["symbol"], (group, m, n, k)
+    for m, n, k, kernel in ((4, 8176, 4096, "k_skinny_gemm"), (4, 8192, 4096, "k_w4_decode"),
+                            (5, 12272, 4096, "k_skinny_gemm"), (5, 12288, 4096, "k_w4_decode"),
+                            (4, 8192, 3072, "k_skinny_gemm"), (4, 8192, 3584, "k_w4_decode"),
+                            (4, 8192, 3712, "k_skinny_gemm"), (1, 8192, 4096, "k_w4_gemv1")):
+        p = w4().pack_uint4((torch.randn(n, k, generator=g) * 0.02).to(cuda), group_size=128)
+        a = torch.randn(m, k, generator=g).to(torch.bfloat16).to(cuda)
+        _, md = w4().int4_linear_a16(a, p, method="dot2", return_kernel=True)
+        assert kernel in md["symbol"] and md["vgpr"] is not None, (m, n, k, md)
 
 
 @pytest.mark.parametrize("m", [1, 2, 3, 4, 16])
