@@ -14,16 +14,10 @@ from test_w4_gpu import act_values, check_product
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("m,n,k", [
-    (17, 130, 1024), (32, 257, 1040), (33, 1, 4096), (64, 300, 12304), (65, 4096, 1152), (200, 1000, 2064),
-    (333, 129, 3072), (1000, 700, 1024), (1030, 140, 1536), (40, 50, 1025),
-])
-@pytest.mark.parametrize("e5,adtype", [(False, torch.bfloat16), (True, torch.float16)])
-def test_fp8_shapes(cuda, m, n, k, e5, adtype):
-    """Row tiles of 32 to 128, splits, a last stage of a few chunks, packed
-    operands (K % 16 != 0), strided rows, scale and bias."""
+def _fp8_case(cuda, m, n, k, e5, adtype):
+    """The call's metadata, its result held to float64: strided activation rows,
+    scale and bias."""
     from rdna2_ops.fp8_weight_gemm_v06 import fp8_weight_gemm
-    case(f"mid fp8 {m}x{n}x{k} e5={e5} {adtype}")
     rng = np.random.default_rng(m * 1000 + n + k)
     codes = rng.integers(0, 256, (n, k)).astype(np.uint8)
     dec = o8.decode_bits(codes, e5)
@@ -34,10 +28,48 @@ def test_fp8_shapes(cuda, m, n, k, e5, adtype):
     md = {}
     y = fp8_weight_gemm(a.to(cuda), codes_tensor(codes, e5, cuda), bias=bias.to(cuda), method="fused_dot2",
                         w_scale=scale.to(cuda), metadata=md)
-    assert md["variant"] == "fp8w_mid" and md["vgpr"] is not None and md["vgpr_spills"] == 0, md
     a64, w64 = a.double().numpy(), o8.decode_bits(codes, e5).astype(np.float64)
     s64, b64 = scale.double().numpy(), bias.double().numpy()
     check(y, (a64 @ w64.T) * s64 + b64, (np.abs(a64) @ np.abs(w64).T) * s64 + np.abs(b64), adtype, "mid fp8")
+    return md
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (17, 130, 1024), (32, 257, 1040), (33, 1, 4096), (64, 300, 12304), (65, 4096, 1152), (200, 1000, 2064),
+    (333, 129, 3072), (1000, 700, 1024), (1030, 140, 1536), (40, 50, 1025),
+])
+@pytest.mark.parametrize("e5,adtype", [(False, torch.bfloat16), (True, torch.float16)])
+def test_fp8_shapes(cuda, m, n, k, e5, adtype):
+    """32-row tiles, splits, a last stage of a few chunks, packed operands (K %
+    16 != 0), strided rows, scale and bias."""
+    case(f"mid fp8 {m}x{n}x{k} e5={e5} {adtype}")
+    md = _fp8_case(cuda, m, n, k, e5, adtype)
+    assert md["variant"] == "fp8w_mid" and md["vgpr"] is not None and md["vgpr_spills"] == 0, md
+
+
+@pytest.mark.parametrize("m,n,k,rows,split", [
+    (300, 515, 1040, 32, False), (17, 130, 2064, 32, True), (333, 3001, 1041, 64, False), (33, 4100, 2064, 64, True),
+    (1000, 2049, 1040, 128, False),
+])
+@pytest.mark.parametrize("e5,adtype", [(False, torch.float16), (True, torch.bfloat16), (False, torch.bfloat16)])
+def test_fp8_tiles(cuda, m, n, k, rows, split, e5, adtype):
+    """Each tile height, unsplit and split, with ragged rows, columns and K."""
+    from rdna2_ops import _lib
+    case(f"mid fp8 tile {m}x{n}x{k} e5={e5} {adtype}")
+    md = _fp8_case(cuda, m, n, k, e5, adtype)
+    assert md["variant"] == "fp8w_mid" and md["vgpr"] is not None and md["vgpr_spills"] == 0, md
+    assert md["launched_tile"][0] == rows, md
+    assert (_lib.library().qg_row_kernel_choice(_lib.CHOICE_FP8, 0, 0, m, n, k) >> 16 > 1) == split
+
+
+@pytest.mark.parametrize("m,n,k", [(2049, 1921, 1040), (2049, 2113, 1025), (1500, 3001, 3080)])
+@pytest.mark.parametrize("e5,adtype", [(False, torch.bfloat16), (True, torch.float16)])
+def test_fp8_smaller_pingpong_grids(cuda, m, n, k, e5, adtype):
+    """The ping-pong kernel below 192 tiles of 256 x 192: partial edge tiles,
+    odd N, K that is no multiple of the stage (operands packed)."""
+    case(f"fp8 ping-pong {m}x{n}x{k} e5={e5} {adtype}")
+    md = _fp8_case(cuda, m, n, k, e5, adtype)
+    assert md["variant"] == ("fp8w_f16_pingpong" if adtype == torch.float16 else "fp8w_bf16_pingpong"), md
 
 
 @pytest.mark.parametrize("rows", [32, 64])
@@ -70,17 +102,10 @@ def test_fp8_values_past_k(cuda):
     assert torch.equal(y.float().cpu(), torch.full((20, n), float(k)))
 
 
-@pytest.mark.parametrize("m,n,k", [(17, 130, 1088), (64, 300, 4096), (65, 4100, 1152), (333, 257, 2048),
-                                   (700, 1030, 1024), (1024, 1100, 3072)])
-@pytest.mark.parametrize("g", o4.GROUPS)
-@pytest.mark.parametrize("sym,order,adtype", [(True, "low", torch.float16), (False, "high", torch.bfloat16)])
-def test_int4_shapes(cuda, m, n, k, g, sym, order, adtype):
-    """Signed INT4 (nk): row tiles, splits, a last stage of fewer groups, both
-    nibble orders, bias. Where the dequant formulation stays the faster one the
-    product is held to the rounded weights' bound by the 1e-2 x RMS bar only."""
+def _int4_case(cuda, m, n, k, g, sym, order, adtype):
+    """The call's metadata, its result held to the exact product of the packed
+    weight: signed INT4 (nk), strided activation rows, bias."""
     from rdna2_ops import int4_weight_gemm_v07 as w4
-    k = k // g * g
-    case(f"mid int4 {m}x{n}x{k} g{g} sym={sym} {order} {adtype}")
     gen = torch.Generator().manual_seed(m + n + k + g)
     w = torch.randn(n, k, generator=gen) * 0.02
     a = torch.randn(m, k + 8, generator=gen).to(adtype)[:, :k]
@@ -90,17 +115,52 @@ def test_int4_shapes(cuda, m, n, k, g, sym, order, adtype):
     av, s = act_values(a), p.scales.cpu().numpy()
     y64 = o4.w4a16_linear(av, cen, s, g, act_values(b))
     y, md = w4.int4_linear_a16(a.to(cuda), p, bias=b.to(cuda), method="dot2", return_kernel=True)
-    if md["variant"] == "w4a16_mid":
-        assert md["vgpr"] is not None and md["vgpr_spills"] == 0, md
-        check_product(y, y64, o4.w4a16_linear(np.abs(av), np.ones_like(cen), s, g), adtype, f"mid int4 {m}x{n}x{k} g{g}")
-    else:
-        err = np.abs(y.float().cpu().numpy() - y64)
-        assert (err <= 1e-2 * np.sqrt(np.mean(y64 ** 2)) + 2.0 ** -8 * np.abs(y64)).all()
+    check_product(y, y64, o4.w4a16_linear(np.abs(av), np.ones_like(cen), s, g), adtype, f"mid int4 {m}x{n}x{k} g{g}")
+    return md
 
 
-@pytest.mark.parametrize("m,n,k", [(20, 140, 14336), (48, 4097, 1152), (96, 520, 4096), (512, 1000, 2048)])
+@pytest.mark.parametrize("m,n,k", [(17, 130, 1088), (64, 300, 4096), (65, 4100, 1152), (333, 257, 2048),
+                                   (700, 1030, 1024), (1024, 1100, 3072)])
+@pytest.mark.parametrize("g", o4.GROUPS)
+@pytest.mark.parametrize("sym,order,adtype", [(True, "low", torch.float16), (False, "high", torch.bfloat16)])
+def test_int4_shapes(cuda, m, n, k, g, sym, order, adtype):
+    """Signed INT4 (nk): splits, a last stage of fewer groups, both nibble
+    orders, bias; 17 rows of a short K stay on the older kernel, to the same
+    bound."""
+    k = k // g * g
+    case(f"mid int4 {m}x{n}x{k} g{g} sym={sym} {order} {adtype}")
+    md = _int4_case(cuda, m, n, k, g, sym, order, adtype)
+    assert md["variant"] == ("w4a16_skinny" if m == 17 else "w4a16_mid"), md
+    assert md["vgpr"] is not None and md["vgpr_spills"] == 0, md
+
+
+INT4_TILES = [(65, 33, 1024, 128, 32, False), (33, 33, 2048, 128, 32, True), (333, 3000, 1024, 128, 64, False),
+              (33, 2049, 6144, 128, 64, True), (1000, 2049, 1024, 128, 128, False), (300, 1537, 4096, 128, 128, True)]
+
+
+@pytest.mark.parametrize("m,n,k,g,rows,split", INT4_TILES + [
+    (90, 33, 1088, 64, 32, False), (33, 33, 2112, 64, 32, True), (333, 3000, 1088, 64, 64, False),
+    (33, 4100, 6144, 64, 64, True), (1000, 2049, 1088, 64, 128, False), (700, 257, 4160, 64, 128, True),
+    (90, 700, 1056, 32, 32, False), (33, 33, 2080, 32, 32, True), (333, 3000, 1056, 32, 64, False),
+    (33, 2049, 4128, 32, 64, True),
+])
+@pytest.mark.parametrize("sym,order,adtype", [(False, "low", torch.float16), (True, "high", torch.bfloat16)])
+def test_int4_tiles(cuda, m, n, k, g, rows, split, sym, order, adtype):
+    """Each tile height of each group size, unsplit and split, with ragged rows,
+    columns and (groups below 128) K."""
+    case(f"mid int4 tile {m}x{n}x{k} g{g} sym={sym} {order} {adtype}")
+    md = _int4_case(cuda, m, n, k, g, sym, order, adtype)
+    assert md["variant"] == "w4a16_mid" and md["vgpr"] is not None and md["vgpr_spills"] == 0, md
+    assert md["tile"][0] == rows and (md["k_splits"] > 1) == split, md
+
+
+@pytest.mark.parametrize("m,n,k,rows,split", [(20, 140, 14336, 32, True), (48, 4097, 1152, 32, False),
+                                              (96, 520, 4096, 32, True), (512, 1000, 2048, 64, True)]
+                         + [(m, n, k, rows, split) for m, n, k, _, rows, split in INT4_TILES])
 @pytest.mark.parametrize("adtype", [torch.float16, torch.bfloat16])
-def test_uint4_shapes(cuda, m, n, k, adtype):
+def test_uint4_shapes(cuda, m, n, k, rows, split, adtype):
+    """uint4 storage (bf16 scales, packed zero points): each tile height,
+    unsplit and split."""
     from rdna2_ops import int4_weight_gemm_v07 as w4
     case(f"mid uint4 {m}x{n}x{k} {adtype}")
     gen = torch.Generator().manual_seed(m + n + k)
@@ -110,7 +170,8 @@ def test_uint4_shapes(cuda, m, n, k, adtype):
     cen = w4.unpack_int4(p, dtype=torch.int8).cpu().numpy().astype(np.int32)
     av, s = act_values(a), p.scales.float().cpu().numpy()
     y, md = w4.int4_linear_a16(a.to(cuda), p, method="dot2", return_kernel=True)
-    assert md["variant"] == "w4a16_mid" and md["vgpr"] is not None
+    assert md["variant"] == "w4a16_mid" and md["vgpr"] is not None and md["vgpr_spills"] == 0, md
+    assert md["tile"][0] == rows and (md["k_splits"] > 1) == split, md
     check_product(y, o4.w4a16_linear(av, cen, s, 128), o4.w4a16_linear(np.abs(av), np.ones_like(cen), s, 128),
                   adtype, f"mid uint4 {m}x{n}x{k}")
 
