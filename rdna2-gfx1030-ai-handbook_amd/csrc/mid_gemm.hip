@@ -1,4 +1,4 @@
-// GEMM of a middling number of activation rows (17 to about a thousand)
+// GEMM of a middling number of activation rows (17 to 2048, K from 1024)
 // against quantized weights on gfx950: out = A @ W^T with W [N, K] int8 (A
 // int8), fp8 or grouped INT4 in the nk layout (A fp16 / bf16).
 //
@@ -8,8 +8,10 @@
 //  * every operand reaches LDS by direct copies in a ring of R slots, R - 1
 //    stages ahead, with one barrier per stage (the copies of stage s + R - 1 go
 //    into the slot that stage s - 1 left, which the barrier shows to be read).
-//    With one stage of lookahead (k_wd_gemm) a stage took 1.7 to 2.1 us, an
-//    L2 / HBM round trip; here 0.5 to 0.7 us (fp8) and 0.6 to 1.3 us (INT4);
+//    With one stage of lookahead (k_wd_gemm, 128 rows) a stage takes 1.4 to 2.2
+//    us, an L2 / HBM round trip; here, with tiles of 32 / 64 / 128 rows, fp8
+//    0.50 / 0.67 / 1.42 us, INT4 0.64 / 0.95 / 1.60 us at group 128, 0.74 / 1.25
+//    / 1.70 at 64, 0.97 / 1.35 at 32, int8 (64 rows) 0.50 us;
 //  * 8 waves, fragments read half a stage ahead of their MFMAs. What is left
 //    of a stage (N 3072, K 12288, M 64, parts removed): fp8 0.73 us, of which
 //    0.60 without the copies (conversions) and 0.57 without the compute (40 to
@@ -470,7 +472,9 @@ hipError_t launch_mid_w4_t(const MidArgs& p, int group, int bm, hipStream_t stre
 
 // Time model (us) behind the choice of tile and split, from a sweep over M 32
 // to 1024 and (N, K) of 1024 x 4096 to 12288 x 3072 and 3072 x 12288 on one
-// box, which it meets within about 10 %: 3.5 us plus the stages of one
+// box, which it meets within about 10 % (over 840 calls, M 17 to 2048, other
+// boxes and weights from HBM take 1.1 to 1.35 times as long, tiles and splits
+// alike): 3.5 us plus the stages of one
 // workgroup times the rounds of 256 workgroups times the time of a stage
 // (128 K elements; 15 % more where rounds overlap); a split adds 2.5 us and
 // its partial tiles at 4 TB/s. A split has to win by 10 %, and its partial tiles
