@@ -444,3 +444,24 @@ def test_int8_gemm_stages_matches_the_gemm(cuda):
     assert (((ext[:, :, 3] - ext[:, :, 0]) % 2 ** 32) > 0).all()
     assert (((ext[:, :, 5] - ext[:, :, 4]) % 2 ** 32) > 0).all()
 
+
+
+@pytest.mark.parametrize("m,n,k", [(8, 3000, 512), (64, 1024, 8192), (300, 3000, 512), (3072, 3072, 128)])
+def test_eager_order_rounds_the_product_to_fp32_first(cuda, m, n, k):
+    """fp16 eager order: f32(acc) * (sa * sb) rounds to fp32, then to fp16. The
+    two differ from one rounding of the product in 6 of 100,000 results; the
+    streaming, split, tiled and ping-pong kernels."""
+    from rdna2_ops.int8_gemm import int8_gemm_dequant
+    case(f"int8 eager fp16 {m}x{n}x{k}")
+    g = torch.Generator().manual_seed(m + n)
+    a = torch.randint(-128, 128, (m, k), generator=g, dtype=torch.int8)
+    w = torch.randint(-128, 128, (n, k), generator=g, dtype=torch.int8)
+    sa, sb = torch.rand(m, generator=g) * 0.02, torch.rand(n, generator=g) * 0.02
+    bias = torch.randn(n, generator=g)
+    ag, wg, sag, sbg = a.to(cuda), w.to(cuda), sa.to(cuda), sb.to(cuda)
+    acc = (ag.double() @ wg.double().T).to(torch.int32).cpu().numpy()  # below 2^53: exact
+    for b in (None, bias):
+        y = int8_gemm_dequant(ag, wg.T, sag, sbg, None if b is None else b.to(cuda), out_dtype=torch.float16,
+                              epilogue_order="eager")
+        ref = o.epilogue_e(acc, sa.numpy(), sb.numpy(), None if b is None else b.numpy(), out="f16")
+        assert np.array_equal(y.float().cpu().numpy(), np.asarray(o.round_to(ref, "f16"), np.float32))
